@@ -87,8 +87,9 @@ int pw4_time_next_kernel(void* start_event, void* stop_event);
 int pw4_observe_next_call(float* y32);
 
 /* Diagnostic, no counterpart in the reference (it is for tests and tuning):
- * writes into buf (len bytes, NUL-terminated) the plan a GEMM call with these
- * arguments would run, e.g. "decode nb=16 wps=256 splits=1 tree=0 win=0 ring=4
+ * writes into buf (len bytes, NUL-terminated) the decode or prefill plan of a
+ * GEMM call with these arguments, which runs unless pw4_medium_plan_describe
+ * names another, e.g. "decode nb=16 wps=256 splits=1 tree=0 win=0 ring=4
  * mt=1 bs=1 px=0" (bs: one scale load per four steps; px: act-order gathered
  * in the kernel's LDS, its permutation columns per thread) or "prefill256
  * rows=128 splits=2 exact=1 khalves=2" (khalves: two K halves per 8-wave
@@ -101,6 +102,14 @@ int pw4_observe_next_call(float* y32);
 #define PW4_LAYOUT_MARLIN 1
 int pw4_plan_describe(int layout, int x_dtype, int scale_dtype, int has_zp, int has_perm, int silu, int64_t M,
                       int64_t N, int64_t K, int64_t group_size, int64_t num_splits, char* buf, size_t len);
+
+/* The same for the medium-M kernel (MARLIN words, or CT words repacked per
+ * call; K and the group size multiples of 64, N of 8): "kwave rows=64 nb=112
+ * splits=1" (rows and columns of a tile, K slices) where the call runs on it,
+ * else "none".  A call whose scales are not 4-byte aligned, or whose workspace
+ * holds only its decode or prefill plan, runs on that plan. */
+int pw4_medium_plan_describe(int layout, int x_dtype, int scale_dtype, int has_zp, int has_perm, int silu, int64_t M,
+                             int64_t N, int64_t K, int64_t group_size, int64_t num_splits, char* buf, size_t len);
 
 /* ABI version of this header: bumped on any incompatible change. */
 int pw4_abi_version(void);

@@ -3,7 +3,9 @@
 #include "pulsar_w4a16.h"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -66,13 +68,14 @@ constexpr size_t kSlotBytes = kZeroRegion - kCounterBytes;
 // environment on every call only when PW4_PLAN_OVERRIDES=1 was set when the
 // process first planned a GEMM; otherwise no call reads the environment (six
 // lookups cost ~0.5 us of host time per call with a typical environment).
-const char* plan_env(const char* name) {
+bool plan_overrides() {
     static const bool enabled = [] {
         const char* e = std::getenv("PW4_PLAN_OVERRIDES");
         return e != nullptr && e[0] == '1';
     }();
-    return enabled ? std::getenv(name) : nullptr;
+    return enabled;
 }
+const char* plan_env(const char* name) { return plan_overrides() ? std::getenv(name) : nullptr; }
 
 // Act-order repack overrides for tuning sweeps and tests: the column block
 // width (8, 16, 32 or 64) and the number of workgroups; unset = heuristic.
@@ -160,6 +163,16 @@ int decode_block_scales_override() {
     const char* e = plan_env("PW4_DECODE_BLOCK_SCALES");
     if (!e) return -1;
     return e[0] == '0' ? 0 : e[0] == '1' ? 1 : -1;
+}
+
+// Whether an override pins a decode or prefill plan: the call then runs on it.
+bool plan_pinned() {
+    for (const char* name : {"PW4_DECODE", "PW4_DECODE_NB", "PW4_DECODE_SPLITS", "PW4_DECODE_WPS", "PW4_DECODE_WIN",
+                             "PW4_DECODE_BLOCK_SCALES", "PW4_DECODE_PERM_LDS", "PW4_PREFILL_TILE", "PW4_PREFILL_ROWS",
+                             "PW4_PREFILL_SPLITS", "PW4_PREFILL_KHALVES", "PW4_PREFILL_EXACT"}) {
+        if (plan_env(name) != nullptr) return true;
+    }
+    return false;
 }
 
 // Windowed decode plans (one unit per workgroup, the activations staged in K
@@ -296,8 +309,101 @@ bool prefer_prefill_tile(int xt, int64_t M, int64_t N, int64_t K, int64_t G, int
     return kModelLow * prefill_us < decode_us;
 }
 
+// Medium-M plan override for tuning sweeps and tests: "0" never, or
+// "<row tiles 1|2>,<columns per tile>,<K slices>" wherever the kernel applies.
+bool kwave_override(int* rt, int* nb, int64_t* splits, bool* never) {
+    const char* e = plan_env("PW4_KWAVE");
+    *never = false;
+    if (!e) return false;
+    long s = 0;
+    if (std::sscanf(e, "%d,%d,%ld", rt, nb, &s) == 3 && (*rt == 1 || *rt == 2) && *nb >= 16 && *nb <= 128 &&
+        *nb % 16 == 0 && s >= 1 && s <= 64) {
+        *splits = s;
+        return true;
+    }
+    *never = true;
+    return false;
+}
+
+// Bytes of CT weights repacked into the workspace: MARLIN words, then fp32 [K/G, N] scales.
+size_t ct_repack_bytes(int64_t N, int64_t K, int64_t G) {
+    return align_up((size_t)round_up(N, kMarlinBN) * round_up(K, kMarlinBK) / 2) + (size_t)(K / G) * N * sizeof(float);
+}
+
+// Plan of the medium-M kernel: row tiles, columns per tile and K slices with the
+// least cost in microseconds.
+struct KwavePlan {
+    int rt = 1, nb = 0;
+    int64_t splits = 1;
+    double us = 0.0;
+};
+
+// The cost model, fitted to graph periods of every (rows, columns, slices) plan
+// on the Llama-3-8B and -70B layers at M = 16..512 on one MI355X (within 10% of
+// the measured period on most of 420 plans):
+//   * a workgroup takes steps * c + e, with steps the 64-K chunks of its busiest
+//     wave and (c, e) by row tiles, 32-column tiles and dtype below (bf16's
+//     exact dequant takes twice the instructions); one workgroup runs per CU;
+//   * the weights, x and y stream at 5.2 TB/s; the two overlap, as the cube root
+//     of the sum of their cubes;
+//   * 4 us of launch, prologue and drain; K slices add 3.5 us and 0.25 per slice
+//     (device-scope partials, the last arriver's reads).
+KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_t max_splits) {
+    constexpr double kStep[2][2][3] = {{{0.52, 0.76, 1.33}, {0.85, 1.17, 1.93}},
+                                       {{0.62, 1.00, 1.85}, {0.90, 1.30, 2.45}}};
+    constexpr double kEnd[2][3] = {{0.6, 0.8, 1.5}, {0.8, 1.4, 2.6}};
+    const double hbm = ((double)N * K * 0.515 + 2.0 * M * (N + K)) / 5.2e6;
+    const int64_t nch = K / 64;
+    KwavePlan best;
+    for (int rt : {1, 2}) {
+        for (int nb : {16, 32, 48, 64, 96, 112, 128}) {
+            const int ci = nb <= 32 ? 0 : nb <= 64 ? 1 : 2;
+            const int64_t tiles = ceil_div(M, 32 * rt) * ceil_div(N, nb);
+            for (int64_t s : {1, 2, 3, 4, 6, 8}) {
+                if (s > max_splits || (s > 1 && s * 8 > nch)) break;
+                const int64_t cps = ceil_div(nch, s);
+                if (s > 1 && ceil_div(nch, cps) != s) continue;  // the same plan as a smaller s
+                const double cu =
+                    (double)ceil_div(tiles * s, (int64_t)cus) *
+                    ((double)ceil_div(cps, 8) * kStep[bf16][rt - 1][ci] + kEnd[rt - 1][ci]);
+                const double us = 4.0 + std::cbrt(hbm * hbm * hbm + cu * cu * cu) + (s > 1 ? 3.5 + 0.25 * (double)s : 0.0);
+                if (best.nb == 0 || us < best.us) best = {rt, nb, s, us};
+            }
+        }
+    }
+    return best;
+}
+
+// What the kernels beside it take, for the choice between them.  The prefill
+// model reads 4 us or more low (launch, ramp and, on K slices, the combine's).
+// The decode kernel at M = 17..32 streams the weights at about 2.5 TB/s behind
+// 4.5 us, and slows down with M (Llama-3-8B, us, decode / K-wave at M = 24 and
+// 32: qkv 10.7 / 9.0 and 11.4 / 9.6, o 7.7 / 8.1 and 9.0 / 8.4, gate_up 26.6 /
+// 18.9 and 29.0 / 19.9, down 22.8 / 14.3 and 24.3 / 14.9).
+double prefill_us(int64_t M, int64_t N, int64_t nchunks, int cus, bool only128) {
+    double us = 0.0;
+    plan_prefill256(M, N, nchunks, cus, only128, 8, &us);
+    return us + 4.0;
+}
+double decode_m32_us(int64_t M, int64_t N, int64_t K) {
+    return (4.5 + (double)N * K / 2.0 / 2.5e6) * (0.7 + 0.0125 * (double)M);
+}
+
+// K slices whose partial tiles stay within a workspace of ws_cap bytes (0: any).
+int64_t max_kwave_splits(int64_t M, int64_t N, int64_t K, size_t ws_cap) {
+    if (ws_cap == 0) return 8;
+    // a slice's partial tiles cover at most (M + 63) x (N + 127) outputs
+    const size_t slice = (size_t)(M + 63) * (N + 127) * 4, fixed = kZeroRegion + (size_t)M * K * 2 + 4 * kAlign;
+    return fixed >= ws_cap ? 1 : std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)((ws_cap - fixed) / slice)));
+}
+
+// Decode batches up to this stay on the decode kernel.
+constexpr int64_t kKwaveMinM = 16;
+
 struct Plan {
     bool decode = false;
+    bool kwave = false;      // medium-M kernel (gemm_kwave.hip)
+    int kw_rt = 1, kw_nb = 0, kw_cps = 0;  // its 32-row tiles, columns per tile and chunks per slice
     bool tree = false;       // decode K slices reduced through the exchange tree
     bool p256 = false;       // prefill on the 256 x 256 tile kernel
     bool p_exact = false;    // ... with exact scaling (fp16 x, 128-row tiles)
@@ -344,9 +450,9 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
     // and 145 / 36, 70B gate_up 218 and 852 / 114, down 210 and 1031 / 74).
     bool decode_ok = M <= 32 && G >= 16 && (G & (G - 1)) == 0;
     const int decode_mode = decode_mode_override();
-    if (decode_mode == 0) decode_ok = false;
+    const int xt = x_dtype == PW4_DTYPE_BF16 ? X_BF16 : X_F16;
     if (decode_ok && decode_mode != 1 && !forced && layout == LAYOUT_MARLIN &&
-        prefer_prefill_tile(x_dtype == PW4_DTYPE_BF16 ? X_BF16 : X_F16, M, N, K, G, cus)) {
+        prefer_prefill_tile(xt, M, N, K, G, cus)) {
         decode_ok = false;
     }
     if (decode_ok) {
@@ -626,7 +732,6 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
         // quant group; with its 128-row tiles and K slices it is measured 20-45%
         // faster than the 128 x 128 kernel at M = 72..160 on every Llama-3-8B
         // layer shape, so it takes every M past the decode kernel's.
-        const int xt = x_dtype == PW4_DTYPE_BF16 ? X_BF16 : X_F16;
         const int tile_pref = prefill_tile_override();
         p.p256 = prefill256_ok(LAYOUT_MARLIN, xt, N, K, G) && tile_pref != 128;
         p.p_exact = p.p256 && xt == X_F16 && prefill_exact_enabled();
@@ -639,10 +744,7 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
         // on CT / decode blocks: 8B gate_up 64.4 and 66.2 / 109 and 109 /
         // 70.2 and 83.4, 70B down 113 and 114 / 271 and 275 / 216 and 346;
         // 8B o 27.1 and 27.4 / 30.7 and 33.5 / 22.8 and 26.3).
-        if (p.p256 && layout == LAYOUT_CT) {
-            p.repack_bytes = align_up((size_t)round_up(N, kMarlinBN) * round_up(K, kMarlinBK) / 2) +
-                             (size_t)(K / G) * N * sizeof(float);
-        }
+        if (p.p256 && layout == LAYOUT_CT) p.repack_bytes = ct_repack_bytes(N, K, G);
         const int64_t tm = p.p256 ? prefill256_tile() : prefill_tile_m();
         const int64_t tn = p.p256 ? prefill256_tile() : prefill_tile_n();
         const int64_t base = ceil_div(M, tm) * ceil_div(N, tn);
@@ -702,6 +804,79 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
     return p;
 }
 
+// The medium-M kernel's plan of a call (kwave false where another kernel is the
+// faster one, or the call is not one it takes).  The CT layout reaches it past
+// the decode range only, repacked; forced K splits and pinned plans never.  A call
+// whose decode or prefill plan needs no workspace takes no K slices here either.
+Plan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
+                       bool has_perm, bool silu, size_t ws_cap, int cus) {
+    Plan p;
+    const int xt = x_dtype == PW4_DTYPE_BF16 ? X_BF16 : X_F16;
+    const int64_t nch = K / 64;
+    KwavePlan kp;
+    bool never = false;
+    if (!kwave_override(&kp.rt, &kp.nb, &kp.splits, &never)) {
+        if (never || plan_pinned()) return p;
+        const double other_us = M <= 32 && (G & (G - 1)) == 0
+                                    ? decode_m32_us(M, N, K)
+                                    : prefill_us(M, N, nch, cus, xt == X_F16 && prefill_exact_enabled());
+        kp = plan_kwave(M, N, K, xt == X_BF16, cus, max_kwave_splits(M, N, K, ws_cap));
+        if (kp.splits > 1 && kp.us < other_us &&
+            make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, 0, silu, ws_cap).workspace() == 0) {
+            kp = plan_kwave(M, N, K, xt == X_BF16, cus, 1);
+        }
+        if (kp.us >= other_us) return p;
+    }
+    const int64_t tiles = ceil_div(M, 32 * kp.rt) * ceil_div(N, kp.nb);
+    if (kp.splits > 1 && tiles > kMaxCounterCols) return p;
+    p.kwave = true;
+    p.kw_rt = kp.rt;
+    p.kw_nb = kp.nb;
+    p.kw_cps = (int)ceil_div(nch, std::min<int64_t>(kp.splits, nch));
+    p.splits = (int)ceil_div(nch, p.kw_cps);
+    p.use_partial = p.splits > 1;
+    if (p.use_partial) {
+        p.partial_bytes = (size_t)tiles * p.splits * kwave_tile_floats(kp.rt, kwave_col_tiles(kp.nb)) * 4;
+    }
+    if (layout == LAYOUT_CT) p.repack_bytes = ct_repack_bytes(N, K, G);
+    if (has_perm) p.xperm_bytes = (size_t)M * K * 2;
+    return p;
+}
+
+// The same with the calling thread's last plans kept (by sizes alone): the
+// search takes about 2 us of host time, and one operator call plans three times.
+Plan make_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
+                     bool has_perm, int64_t num_splits, bool silu, size_t ws_cap) {
+    if (num_splits >= 1 || M <= kKwaveMinM || (layout != LAYOUT_MARLIN && M <= 32) || !kwave_ok(N, K, G, 4)) return {};
+    const int cus = cu_count();
+    if (plan_overrides()) {  // they may change from call to call
+        return search_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, silu, ws_cap, cus);
+    }
+    using Key = std::array<int64_t, 7>;
+    const Key key{M, N, K, G, (int64_t)ws_cap, cus,
+                  layout | x_dtype << 4 | stype << 8 | (int)zp << 12 | (int)has_perm << 13 | (int)silu << 14};
+    struct Entry {
+        Key key{-1};
+        Plan plan;
+    };
+    constexpr size_t kEntries = 64;
+    static thread_local Entry table[kEntries];
+    Entry& e = table[(size_t)(M * 31 + N / 8 * 7 + K / 64 * 3 + key[6]) % kEntries];
+    if (e.key != key) {
+        e.plan = search_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, silu, ws_cap, cus);
+        e.key = key;
+    }
+    return e.plan;
+}
+
+// Workspace bytes of a call: for whichever of its two plans runs.
+size_t call_workspace(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
+                      bool has_perm, int64_t num_splits, bool silu = false, size_t ws_cap = 0) {
+    return std::max(
+        make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, num_splits, silu, ws_cap).workspace(),
+        make_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, num_splits, silu, ws_cap).workspace());
+}
+
 int check_common(int64_t M, int64_t N, int64_t K, int64_t G, int x_dtype) {
     if (M < 0 || N < 0 || K < 0) return PW4_ERR_ARG;
     if (x_dtype != PW4_DTYPE_F16 && x_dtype != PW4_DTYPE_BF16) return PW4_ERR_ARG;
@@ -719,8 +894,14 @@ int run_gemm(int layout, const void* x, int x_dtype, const uint32_t* w, const vo
              bool silu = false, size_t ws_cap = 0) {
     // x and the weight words are read as 16-byte vectors
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) return PW4_ERR_ARG;
-    const Plan p = make_plan(layout, x_dtype, stype, qzeros != nullptr, M, N, K, G, perm != nullptr, num_splits, silu,
+    // the medium-M kernel copies the scales as 4-byte words and needs its own scratch;
+    // without either the call runs on its decode or prefill plan
+    Plan p = make_kwave_plan(layout, x_dtype, stype, qzeros != nullptr, M, N, K, G, perm != nullptr, num_splits, silu,
                              ws_cap);
+    if (!p.kwave || (layout == LAYOUT_MARLIN && (reinterpret_cast<uintptr_t>(scales) & 3) != 0) ||
+        (p.workspace() > 0 && (workspace == nullptr || ws_bytes < p.workspace()))) {
+        p = make_plan(layout, x_dtype, stype, qzeros != nullptr, M, N, K, G, perm != nullptr, num_splits, silu, ws_cap);
+    }
     if (p.workspace() > 0 && (workspace == nullptr || ws_bytes < p.workspace())) return PW4_ERR_WORKSPACE;
     char* ws = reinterpret_cast<char*>(workspace);
     int32_t* counters = p.workspace() ? reinterpret_cast<int32_t*>(ws) : nullptr;
@@ -799,6 +980,27 @@ int run_gemm(int layout, const void* x, int x_dtype, const uint32_t* w, const vo
         a.spr_recip = (uint32_t)(((uint64_t{1} << 32) + (uint64_t)(a.kwin / 8 + 1) - 1) / (uint64_t)(a.kwin / 8 + 1));
         e = launch_decode(layout, xt, stype, qzeros != nullptr, dc, a, stream, ev);
         if (e != hipSuccess) return hip_fail(e);
+    } else if (p.kwave) {
+        KwaveArgs a{};
+        a.x = xin;
+        a.w = w;
+        a.scales = scales;
+        a.qzeros = qzeros;
+        a.y = y_gemm;
+        a.partial = p.use_partial ? partial : nullptr;
+        a.counters = counters;
+        a.y32 = silu ? nullptr : ev.y32;
+        a.M = (int)M;
+        a.N = (int)N;
+        a.K = (int)K;
+        a.G = (int)G;
+        a.nb = p.kw_nb;
+        a.splits = p.splits;
+        a.chunks_per_split = p.kw_cps;
+        a.nchunks = (int)(K / 64);
+        a.silu = silu ? 1 : 0;
+        e = launch_kwave(xt, stype, qzeros != nullptr, p.kw_rt, a, stream, ev);
+        if (e != hipSuccess) return hip_fail(e);
     } else {
         PrefillArgs a{};
         a.x = xin;
@@ -828,7 +1030,7 @@ int run_gemm(int layout, const void* x, int x_dtype, const uint32_t* w, const vo
                    : launch_prefill(layout, xt, stype, qzeros != nullptr, a, stream, ev);
         if (e != hipSuccess) return hip_fail(e);
     }
-    if (p.use_partial && !p.decode) {
+    if (p.use_partial && !p.decode && !p.kwave) {
         e = silu ? launch_combine_silu(partial, reinterpret_cast<uint16_t*>(y), M, N, p.splits, xt, stream)
                  : launch_combine(partial, reinterpret_cast<uint16_t*>(y), M * N, p.splits, xt, stream, ev.y32);
         if (e != hipSuccess) return hip_fail(e);
@@ -974,6 +1176,23 @@ int pw4_plan_describe(int layout, int x_dtype, int scale_dtype, int has_zp, int 
     return n < 0 || (size_t)n >= len ? PW4_ERR_ARG : PW4_OK;
 }
 
+int pw4_medium_plan_describe(int layout, int x_dtype, int scale_dtype, int has_zp, int has_perm, int silu, int64_t M,
+                             int64_t N, int64_t K, int64_t group_size, int64_t num_splits, char* buf, size_t len) {
+    if (layout != PW4_LAYOUT_CT && layout != PW4_LAYOUT_MARLIN) return PW4_ERR_ARG;
+    const int rc = check_common(M, N, K, group_size, x_dtype);
+    if (rc != PW4_OK) return rc;
+    if (num_splits < 0 || buf == nullptr || len == 0) return PW4_ERR_ARG;
+    if (scale_dtype != PW4_DTYPE_F32 && scale_dtype != PW4_DTYPE_F16) return PW4_ERR_ARG;
+    if (M == 0 || N == 0) return PW4_ERR_SHAPE;
+    const Plan p = make_kwave_plan(layout == PW4_LAYOUT_MARLIN ? LAYOUT_MARLIN : LAYOUT_CT, x_dtype,
+                                   scale_dtype == PW4_DTYPE_F32 ? S_F32 : S_F16, has_zp != 0, M, N, K, group_size,
+                                   has_perm != 0, num_splits, silu != 0, 0);
+    const int n = p.kwave ? std::snprintf(buf, len, "kwave rows=%d nb=%d splits=%d%s", 32 * p.kw_rt, p.kw_nb, p.splits,
+                                          p.repack_bytes ? " repack" : "")
+                          : std::snprintf(buf, len, "none");
+    return n < 0 || (size_t)n >= len ? PW4_ERR_ARG : PW4_OK;
+}
+
 int pw4_abi_version(void) { return PW4_ABI_VERSION; }
 
 int64_t pw4_marlin_words(int64_t N, int64_t K) {
@@ -1009,8 +1228,8 @@ int pw4_repack_w4a16(const int32_t* weight_packed, const void* weight_scale, int
 size_t pw4_gemm_w4a16_workspace_size(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t num_splits) {
     if (check_common(M, N, K, group_size, PW4_DTYPE_F16) != PW4_OK || M == 0 || N == 0) return 0;
     // the plan may differ by activation dtype (LDS budget): size for both
-    return std::max(make_plan(LAYOUT_CT, PW4_DTYPE_F16, S_F32, false, M, N, K, group_size, false, num_splits).workspace(),
-                    make_plan(LAYOUT_CT, PW4_DTYPE_BF16, S_F32, false, M, N, K, group_size, false, num_splits).workspace());
+    return std::max(call_workspace(LAYOUT_CT, PW4_DTYPE_F16, S_F32, false, M, N, K, group_size, false, num_splits),
+                    call_workspace(LAYOUT_CT, PW4_DTYPE_BF16, S_F32, false, M, N, K, group_size, false, num_splits));
 }
 
 int pw4_gemm_w4a16(const void* x, int x_dtype, const int32_t* weight_packed, const float* weight_scale, void* y,
@@ -1031,8 +1250,8 @@ size_t pw4_gemm_w4a16_marlin_workspace_size(int64_t M, int64_t N, int64_t K, int
                                             int64_t num_splits) {
     if (check_common(M, N, K, group_size, PW4_DTYPE_F16) != PW4_OK || M == 0 || N == 0) return 0;
     return std::max(
-        make_plan(LAYOUT_MARLIN, PW4_DTYPE_F16, S_F16, true, M, N, K, group_size, has_perm != 0, num_splits).workspace(),
-        make_plan(LAYOUT_MARLIN, PW4_DTYPE_BF16, S_F16, true, M, N, K, group_size, has_perm != 0, num_splits).workspace());
+        call_workspace(LAYOUT_MARLIN, PW4_DTYPE_F16, S_F16, true, M, N, K, group_size, has_perm != 0, num_splits),
+        call_workspace(LAYOUT_MARLIN, PW4_DTYPE_BF16, S_F16, true, M, N, K, group_size, has_perm != 0, num_splits));
 }
 
 int pw4_gemm_w4a16_marlin(const void* x, int x_dtype, const int32_t* weight_marlin, const void* scales,
@@ -1065,10 +1284,9 @@ int pw4_gemm_w4a16_marlin_noalloc(const void* x, int x_dtype, const int32_t* wei
     if (M == 0 || N == 0) return PW4_OK;
     if (!x || !weight_marlin || !scales || !y) return PW4_ERR_ARG;
     // the plan run_gemm will make, sized before anything is launched
-    const size_t need = make_plan(LAYOUT_MARLIN, x_dtype, scale_dtype == PW4_DTYPE_F32 ? S_F32 : S_F16,
+    const size_t need = call_workspace(LAYOUT_MARLIN, x_dtype, scale_dtype == PW4_DTYPE_F32 ? S_F32 : S_F16,
                                   qzeros != nullptr, M, N, K, group_size, perm != nullptr, num_splits, false,
-                                  kStaticScratchBytes)
-                            .workspace();
+                                  kStaticScratchBytes);
     if (need > kStaticScratchBytes) return PW4_ERR_WORKSPACE;
     const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     void* ws = nullptr;
@@ -1085,8 +1303,8 @@ int pw4_gemm_w4a16_marlin_noalloc(const void* x, int x_dtype, const int32_t* wei
 size_t pw4_gemm_w4a16_silu_mul_workspace_size(int64_t M, int64_t N, int64_t K, int64_t group_size, int has_perm) {
     if (check_common(M, N, K, group_size, PW4_DTYPE_F16) != PW4_OK || M == 0 || N == 0 || N % 16 != 0) return 0;
     return std::max(
-        make_plan(LAYOUT_MARLIN, PW4_DTYPE_F16, S_F16, true, M, N, K, group_size, has_perm != 0, 0, true).workspace(),
-        make_plan(LAYOUT_MARLIN, PW4_DTYPE_BF16, S_F16, true, M, N, K, group_size, has_perm != 0, 0, true).workspace());
+        call_workspace(LAYOUT_MARLIN, PW4_DTYPE_F16, S_F16, true, M, N, K, group_size, has_perm != 0, 0, true),
+        call_workspace(LAYOUT_MARLIN, PW4_DTYPE_BF16, S_F16, true, M, N, K, group_size, has_perm != 0, 0, true));
 }
 
 int pw4_gemm_w4a16_silu_mul(const void* x, int x_dtype, const int32_t* weight_marlin, const void* scales,

@@ -182,6 +182,46 @@ int64_t prefill256_tail_cols(int64_t M, int64_t N, int cus, double* waves);
 hipError_t launch_prefill256(int xtype, int stype, bool zp, const PrefillArgs& a, hipStream_t stream,
                              KernelEvents ev = {});
 
+// Medium-M GEMM (MARLIN layout, K and the group size multiples of 64): tiles
+// of 32 * rt rows by nb columns, eight K waves per workgroup, K slices across
+// workgroups summed by the last to arrive.
+struct KwaveArgs {
+    const uint16_t* x;       // [M, K] (already act-order permuted when needed)
+    const uint32_t* w;
+    const void* scales;      // [K/G, N], 4-byte aligned
+    const uint32_t* qzeros;  // [K/G, N/8] or null
+    uint16_t* y;             // [M, N], or [M, N/2] with silu
+    float* partial;          // splits > 1: [tiles, splits, kwave_tile_floats] fp32, else null
+    int32_t* counters;       // splits > 1: [tiles] arrival counters (zero on entry, left zero)
+    float* y32;              // [M, N] fp32 copy of the output before rounding, or null (not with silu)
+    int M, N, K, G;
+    int nb;                  // columns per tile: a multiple of 16 up to 128
+    int splits;              // K slices
+    int chunks_per_split;    // 64-K chunks per slice
+    int nchunks;             // K / 64
+    int silu;
+    // filled by launch_kwave
+    int Kg, cpg;             // quant groups; 64-K chunks per group
+    uint32_t cpg_recip;      // ceil(2^32 / cpg)
+    int ncols;               // columns present in the weight layout
+    uint32_t w_bytes;
+    int num_m, num_n;        // row and column tiles
+    int run_log2;            // log2 of the consecutive chunks a wave takes
+    NibbleMasks masks;
+};
+// Whether the kernel takes these sizes (sbytes: bytes of a scale).
+bool kwave_ok(int64_t N, int64_t K, int64_t G, int sbytes);
+// fp32 values of one partial tile (rt 1 or 2; ct = 32-column tiles: 1, 2 or 4).
+int kwave_tile_floats(int rt, int ct);
+// 32-column tiles the kernel for nb columns is built for (1, 2 or 4).
+constexpr int kwave_col_tiles(int nb) { return nb <= 32 ? 1 : nb <= 64 ? 2 : 4; }
+using KwaveFn = void (*)(const KwaveArgs);
+KwaveFn kwave_f16(int stype, bool zp, int rt, int ct);
+KwaveFn kwave_bf16(int stype, bool zp, int rt, int ct);
+constexpr int kKwaveThreads = 512;
+hipError_t launch_kwave(int xtype, int stype, bool zp, int rt, const KwaveArgs& a, hipStream_t stream,
+                        KernelEvents ev = {});
+
 // x_out[m, j] = x[m, perm[j]].  staged: 1 stages each source row in LDS (when
 // K * 2 <= 64 KB and the pointers are 16-byte aligned), 0 reads it directly,
 // -1 picks staged for M > kGatherStagedMinM.

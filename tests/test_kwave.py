@@ -1,0 +1,169 @@
+"""The medium-M GEMM (gemm_kwave.h): eight K waves per tile, sums through LDS, K slices summed by
+the last workgroup to arrive.
+
+PW4_KWAVE="<row tiles>,<columns>,<slices>" pins its tile, so that every edge is reached: one and
+two 32-row tiles, full and ragged; 16 to 128 columns on 1, 2 and 4 column tiles, with tiles that
+straddle the 64-column weight blocks; waves without a chunk, uneven waves, several ring rounds;
+slices of unequal length.  The bars are those of every GEMM test (w4a16_case), against the fp32
+oracle.
+"""
+
+import ctypes
+import os
+
+import numpy as np
+import pytest
+import torch
+
+import pulsar_amd
+from pulsar_amd import ops
+from pw4_capi import DTYPE_BF16, DTYPE_F16
+from w4a16_case import baseline_case, check
+
+
+def describe(m, k, n, g=128, dtype=DTYPE_F16, layout=1, perm=0, splits=0):
+    lib = pulsar_amd.capi()
+    lib.pw4_medium_plan_describe.argtypes = [ctypes.c_int] * 6 + [ctypes.c_int64] * 5 + [ctypes.c_char_p, ctypes.c_size_t]
+    buf = ctypes.create_string_buffer(160)
+    rc = lib.pw4_medium_plan_describe(layout, dtype, DTYPE_F16, 0, perm, 0, m, n, k, g, splits, buf, len(buf))
+    assert rc == 0, rc
+    return buf.value.decode()
+
+
+@pytest.fixture
+def pin():
+    old = os.environ.pop("PW4_KWAVE", None)
+
+    def set_(v):
+        if v is None:
+            os.environ.pop("PW4_KWAVE", None)
+        else:
+            os.environ["PW4_KWAVE"] = v
+
+    yield set_
+    set_(old)
+
+
+def _run(c, g, sdtype, act, sym, offset=0):
+    g_idx = torch.from_numpy(c.g_idx).cuda() if act else None
+    wm, perm = ops.repack_w4a16_gptq(c.qweight(), g_idx, g)
+    s = torch.from_numpy(np.ascontiguousarray(c.scale_nk.T)).to(sdtype).cuda()
+    if offset:  # the same values at an address that is not a multiple of four
+        buf = torch.empty(s.numel() + offset, dtype=sdtype, device="cuda")
+        buf[offset:].copy_(s.reshape(-1))
+        s = buf[offset:].view(s.shape)
+    return ops.gemm_w4a16_gptq(c.x, wm, s, None if sym else c.qzeros(), perm if act else None, g)
+
+
+# (pin, m, n, k, g)
+CASES = [
+    ("1,16,1", 17, 64, 64, 64),       # one chunk: seven waves without one
+    ("1,32,1", 32, 96, 512, 64),      # one chunk a wave
+    ("1,48,1", 31, 200, 1088, 64),    # 17 chunks; tiles straddle the 64-column blocks, ragged N
+    ("1,112,1", 33, 456, 2304, 256),  # two row tiles of 32, the second of one row; 36 chunks
+    ("1,128,3", 20, 1000, 4096, 128),  # 22 + 22 + 20 chunks
+    ("2,16,2", 64, 128, 1024, 128),
+    ("2,64,1", 65, 320, 4160, 64),    # a second row tile of one row; 65 chunks
+    ("2,96,1", 63, 520, 768, 128),
+    ("2,112,5", 130, 904, 2560, 128),
+    ("2,128,8", 48, 136, 8192, 128),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sdtype,sym,act", [(torch.float16, True, False), (torch.float32, False, True)])
+@pytest.mark.parametrize("plan,m,n,k,g", CASES)
+def test_kwave_plans(pin, plan, m, n, k, g, dtype, sdtype, sym, act):
+    c = baseline_case(m, n, k, g, dtype=dtype, seed=m * 3 + n, symmetric=sym, act_order=act)
+    pin(plan)
+    y = _run(c, g, sdtype, act, sym)
+    check(y, c.y_ref, dtype, f"{plan} m={m} n={n} k={k} g={g} {dtype}")
+    for _ in range(3):  # the counters are left zero, and the sum does not depend on arrival
+        assert torch.equal(_run(c, g, sdtype, act, sym), y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("plan", ["1,64,1", "2,128,2"])
+def test_zero_and_negative_scales(pin, plan, dtype):
+    """A group whose scale is zero adds nothing (wherever it lies in a wave's chunks), and
+    negative scales are as good as positive ones."""
+    m, n, k, g = 40, 256, 2048, 128
+    c = baseline_case(m, n, k, g, dtype=dtype, seed=5)
+    rng = np.random.default_rng(7)
+    s = c.scale_nk * np.where(rng.random(c.scale_nk.shape) < 0.5, -1, 1)
+    s[rng.random(s.shape) < 0.4] = 0.0
+    s[3] = 0.0       # a column without any weight
+    s[5, 1:] = 0.0   # the first group alone
+    s[6, :-1] = 0.0  # the last group alone
+    c.scale_nk = s.astype(np.float32)
+    w = (c.u.astype(np.float32) - 8) * np.repeat(c.scale_nk, g, axis=1)
+    ref = c.x.float().cpu().numpy() @ w.T
+    pin(plan)
+    y = _run(c, g, torch.float32, False, True)
+    check(y, ref, dtype, f"{plan} {dtype}")
+    assert (y[:, 3] == 0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_infinite_and_nan_rows_stay_in_their_rows(pin, dtype):
+    m, n, k, g = 48, 192, 1024, 128
+    c = baseline_case(m, n, k, g, dtype=dtype, seed=9)
+    c.x[7, 100] = float("inf")
+    c.x[40, 900] = float("nan")
+    pin("2,64,2")
+    y = _run(c, g, torch.float16, False, True).float()
+    keep = torch.ones(m, dtype=torch.bool)
+    keep[[7, 40]] = False
+    check(y[keep].to(dtype), c.y_ref[keep.numpy()], dtype, "the other rows")
+    assert y[40].isnan().all()
+    u = torch.from_numpy(c.u[:, 100].astype(np.int64)).cuda() - 8  # inf * weight: its sign, or NaN for 0
+    assert torch.equal(y[7][u > 0], torch.full_like(y[7][u > 0], float("inf")))
+    assert torch.equal(y[7][u < 0], torch.full_like(y[7][u < 0], float("-inf")))
+    assert y[7][u == 0].isnan().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,g", [(32, 6144, 4096, 128), (100, 520, 4160, 64)])
+def test_default_plan_and_unaligned_scales(pin, m, n, k, g, dtype):
+    """The plan the library picks by itself, and the call it does not take: fp16 scales at an odd
+    2-byte address run on the decode or prefill plan, with the same result up to rounding."""
+    c = baseline_case(m, n, k, g, dtype=dtype, seed=m)
+    pin(None)
+    assert describe(m, k, n, g, DTYPE_BF16 if dtype == torch.bfloat16 else DTYPE_F16).startswith("kwave")
+    for offset in (0, 1):
+        check(_run(c, g, torch.float16, False, True, offset), c.y_ref, dtype, f"m={m} offset={offset}")
+
+
+@pytest.mark.parametrize("m,k,n,kwave", [
+    # us on MI355X, graph periods, fp16 x: K-wave / the decode or prefill plan
+    (24, 4096, 6144, True),    # 9.0 / 10.7
+    (24, 4096, 4096, False),   # 8.1 / 7.7
+    (32, 4096, 28672, True),   # 19.9 / 29.0
+    (32, 14336, 4096, True),   # 14.9 / 24.3
+    (64, 4096, 4096, True),    # 9.2 / 19.0
+    (128, 14336, 4096, True),  # 25.7 / 35.3
+    (256, 4096, 6144, True),   # 20.9 / 28.3
+    (256, 4096, 28672, False),  # 85 / 65.6
+    (4096, 4096, 28672, False),
+    (16, 4096, 28672, False),  # 18.2 / 16.0
+])
+def test_planner(pin, m, k, n, kwave):
+    pin(None)
+    assert (describe(m, k, n) != "none") == kwave, describe(m, k, n)
+
+
+def test_planner_keeps_what_the_kernel_does_not_take(pin):
+    pin(None)
+    assert describe(64, 4096, 4096, splits=2) == "none"   # a forced K split
+    assert describe(64, 4096, 4096, g=32) == "none"       # groups inside a chunk
+    assert describe(64, 4128, 4096, g=32) == "none"
+    assert describe(64, 4096, 4100) == "none"             # N % 8
+    assert describe(64, 0, 4096) == "none"
+    assert describe(32, 4096, 4096, layout=0) == "none"   # packed words at decode sizes
+    assert describe(64, 4096, 4096, layout=0).endswith("repack")
+    # K / 64 below eight chunks still has a plan
+    assert describe(2000, 64, 512, g=64) in ("none", "kwave rows=64 nb=128 splits=1")
