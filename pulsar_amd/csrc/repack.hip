@@ -436,12 +436,19 @@ __global__ __launch_bounds__(kPermThreads) void repack_gptq_perm_kernel(const ui
 // span again and writes row k at the group's count of earlier rows (earlier
 // waves, earlier steps, lower lanes, the lane's earlier entries).  A lane
 // loads its entries of kGidxBatch steps at once: the walks are bound by their
-// memory round trips.
-template <bool VEC, int kGidxWaves, int kGidxBatch>
+// memory round trips.  ONE: a wave's span is one batch, whose matches stay in
+// registers, so pass 2 has no round trip of its own (K = 14336: 10.6 -> 6.9 us).
+// With one workgroup more than there are groups (hist_groups != 0), the last one
+// counts all groups in LDS and stores the status, so that no kernel has to clear
+// it first; else the groups' workgroups OR their findings into a cleared status.
+template <bool VEC, int kGidxWaves, int kGidxBatch, bool ONE>
 __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_t* __restrict__ g_idx,
                                                                     int32_t* __restrict__ perm,
-                                                                    int32_t* __restrict__ status, int K, int G) {
+                                                                    int32_t* __restrict__ status, int K, int G,
+                                                                    int hist_groups) {
     constexpr int EPL = VEC ? 4 : 1, kStep = 64 * EPL;
+    static_assert(kGidxBatch * EPL <= 32, "a batch's matches are one word per lane");
+    extern __shared__ int hist[];
     __shared__ int wave_cnt[kGidxWaves];
     const int g = blockIdx.x;
     const int Kg = K / G;
@@ -449,9 +456,8 @@ __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_
     const int span = (K + kGidxWaves * kStep - 1) / (kGidxWaves * kStep) * kStep;
     const int k_begin = wave * span, k_end = min(k_begin + span, K);  // VEC: K % 4 == 0, whole 4-entry runs
     const uint64_t below = (1ull << lane) - 1ull;
-    // one batch of kGidxBatch steps: the group's rows among entries k0 + kStep b + EPL lane + j
-    auto batch = [&](int k0, bool (&mine)[kGidxBatch][EPL]) {
-        int gv[kGidxBatch][EPL];
+    // entries k0 + kStep b + EPL lane + j of one batch of kGidxBatch steps (-1 past the span)
+    auto load = [&](int k0, int (&gv)[kGidxBatch][EPL]) {
 #pragma unroll
         for (int b = 0; b < kGidxBatch; ++b) {
             const int k = k0 + b * kStep + lane * EPL;
@@ -465,23 +471,57 @@ __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_
                 gv[b][0] = k < k_end ? g_idx[k] : -1;
             }
         }
+    };
+    if (g == Kg) {  // the counting workgroup
+        for (int i = tid; i < Kg; i += 64 * kGidxWaves) hist[i] = 0;
+        if (tid == 0) wave_cnt[0] = 0;
+        __syncthreads();
+        bool bad_id = false;
+        for (int k0 = k_begin; k0 < k_end; k0 += kStep * kGidxBatch) {
+            int gv[kGidxBatch][EPL];
+            load(k0, gv);
+#pragma unroll
+            for (int b = 0; b < kGidxBatch; ++b)
+#pragma unroll
+                for (int j = 0; j < EPL; ++j) {
+                    if (k0 + b * kStep + lane * EPL + j >= k_end) continue;
+                    if (gv[b][j] < 0 || gv[b][j] >= Kg) {
+                        bad_id = true;
+                    } else {
+                        atomicAdd(&hist[gv[b][j]], 1);
+                    }
+                }
+        }
+        __syncthreads();
+        int st = bad_id ? 2 : 0;
+        for (int i = tid; i < Kg; i += 64 * kGidxWaves) st |= hist[i] != G ? 1 : 0;
+        if (st) atomicOr(&wave_cnt[0], st);
+        __syncthreads();
+        if (tid == 0) *status = wave_cnt[0];
+        return;
+    }
+    // bit b * EPL + j: whether that entry of a batch is the group's
+    auto batch = [&](int k0) {
+        int gv[kGidxBatch][EPL];
+        load(k0, gv);
+        uint32_t mine = 0;
 #pragma unroll
         for (int b = 0; b < kGidxBatch; ++b)
 #pragma unroll
             for (int j = 0; j < EPL; ++j) {
                 const int k = k0 + b * kStep + lane * EPL + j;
-                if (g == 0 && k < k_end && (gv[b][j] < 0 || gv[b][j] >= Kg)) atomicOr(status, 2);
-                mine[b][j] = k < k_end && gv[b][j] == g;
+                if (hist_groups == 0 && g == 0 && k < k_end && (gv[b][j] < 0 || gv[b][j] >= Kg)) atomicOr(status, 2);
+                mine |= (uint32_t)(k < k_end && gv[b][j] == g) << (b * EPL + j);
             }
+        return mine;
     };
     int count = 0;
+    uint32_t first = 0;
     for (int k0 = k_begin; k0 < k_end; k0 += kStep * kGidxBatch) {
-        bool mine[kGidxBatch][EPL];
-        batch(k0, mine);
+        const uint32_t mine = batch(k0);
+        if constexpr (ONE) first = mine;
 #pragma unroll
-        for (int b = 0; b < kGidxBatch; ++b)
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) count += __popcll(__ballot(mine[b][j]));
+        for (int i = 0; i < kGidxBatch * EPL; ++i) count += __popcll(__ballot((mine >> i) & 1u));
     }
     if (lane == 0) wave_cnt[wave] = count;
     __syncthreads();
@@ -492,27 +532,27 @@ __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_
         total += wave_cnt[w];
     }
     for (int k0 = k_begin; k0 < k_end; k0 += kStep * kGidxBatch) {
-        bool mine[kGidxBatch][EPL];
-        batch(k0, mine);
+        const uint32_t mine = ONE ? first : batch(k0);
 #pragma unroll
         for (int b = 0; b < kGidxBatch; ++b) {
             int lower = 0, step = 0;
 #pragma unroll
             for (int j = 0; j < EPL; ++j) {
-                const uint64_t mask = __ballot(mine[b][j]);
+                const uint64_t mask = __ballot((mine >> (b * EPL + j)) & 1u);
                 lower += __popcll(mask & below);
                 step += __popcll(mask);
             }
             int at = pos + lower;
 #pragma unroll
             for (int j = 0; j < EPL; ++j) {
-                if (mine[b][j] && at < G) perm[(int64_t)g * G + at] = k0 + b * kStep + lane * EPL + j;
-                at += mine[b][j] ? 1 : 0;
+                const bool m = (mine >> (b * EPL + j)) & 1u;
+                if (m && at < G) perm[(int64_t)g * G + at] = k0 + b * kStep + lane * EPL + j;
+                at += m ? 1 : 0;
             }
             pos += step;
         }
     }
-    if (tid == 0 && total != G) atomicOr(status, 1);
+    if (hist_groups == 0 && tid == 0 && total != G) atomicOr(status, 1);
 }
 
 __global__ __launch_bounds__(64) void clear_status_kernel(int32_t* __restrict__ status) {
@@ -637,21 +677,37 @@ hipError_t launch_repack_gptq(const uint32_t* qweight, const int32_t* perm, uint
 
 
 hipError_t launch_gidx_perm(const int32_t* g_idx, int32_t* perm, int32_t* status, int K, int G, hipStream_t stream) {
-    // the status word is cleared by a kernel rather than a memset, so that a
-    // caller capturing the stream into a graph records a kernel node
-    hipLaunchKernelGGL(clear_status_kernel, dim3(1), dim3(64), 0, stream, status);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || K == 0) return e;
+    const int groups = K > 0 ? K / G : 0;
+    // The status from a counting workgroup beside the groups' where its counters fit
+    // in LDS, in place of a launch that clears it first (1.5 us and a gap).
+    const int hist = groups > 0 && groups <= 16384 ? groups : 0;
+    if (hist == 0) {
+        // cleared by a kernel rather than a memset, so that a caller capturing the
+        // stream into a graph records a kernel node
+        hipLaunchKernelGGL(clear_status_kernel, dim3(1), dim3(64), 0, stream, status);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || K == 0) return e;
+    }
+    const dim3 grid(groups + (hist ? 1 : 0));
+    const size_t lds = (size_t)hist * 4;
+    auto go = [&](auto fn, int threads) {
+        hipLaunchKernelGGL(fn, grid, dim3(threads), lds, stream, g_idx, perm, status, K, G, hist);
+    };
     // Past K = 4096, eight waves with 16-byte loads where g_idx is 16-byte aligned
     // and K holds whole 4-entry runs (K = 14336: 17.4 -> 9.6 us, 28672: 29.2 ->
     // 18.1 us against four waves of single entries); up to K = 4096 four waves
-    // of single entries are faster (5.2 against 7.8 us at 4096).
+    // of single entries are faster (5.2 against 7.8 us at 4096).  Spans of one
+    // batch (K = 4096, and up to 16384 with 16-byte loads) keep it in registers.
     if ((reinterpret_cast<uintptr_t>(g_idx) & 15) == 0 && K % 4 == 0 && K > 4096) {
-        hipLaunchKernelGGL((gidx_perm_kernel<true, 8, 8>), dim3(K / G), dim3(512), 0, stream, g_idx, perm, status, K,
-                           G);
+        if (K <= 8 * 64 * 4 * 8) {
+            go(gidx_perm_kernel<true, 8, 8, true>, 512);
+        } else {
+            go(gidx_perm_kernel<true, 8, 8, false>, 512);
+        }
+    } else if (K <= 4 * 64 * 16) {
+        go(gidx_perm_kernel<false, 4, 16, true>, 256);
     } else {
-        hipLaunchKernelGGL((gidx_perm_kernel<false, 4, 16>), dim3(K / G), dim3(256), 0, stream, g_idx, perm, status,
-                           K, G);
+        go(gidx_perm_kernel<false, 4, 16, false>, 256);
     }
     return hipGetLastError();
 }

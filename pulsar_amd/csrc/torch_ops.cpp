@@ -95,6 +95,26 @@ at::Tensor workspace(size_t bytes, const at::Tensor& like) {
     return w.buf;
 }
 
+// A point of a stream that the host can wait for.
+class StreamPoint {
+   public:
+    StreamPoint() = default;
+    StreamPoint(const StreamPoint&) = delete;
+    StreamPoint& operator=(const StreamPoint&) = delete;
+    ~StreamPoint() {
+        if (ev_ != nullptr) (void)hipEventDestroy(ev_);
+    }
+    void record(hipStream_t stream) {
+        check(hipEventCreateWithFlags(&ev_, hipEventDisableTiming));
+        check(hipEventRecord(ev_, stream));
+    }
+    void wait() { check(hipEventSynchronize(ev_)); }
+
+   private:
+    static void check(hipError_t e) { TORCH_CHECK(e == hipSuccess, "HIP event: ", hipGetErrorString(e)); }
+    hipEvent_t ev_ = nullptr;
+};
+
 void* ptr_or_null(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 at::Tensor gemm_w4a16_run(const at::Tensor& x, const at::Tensor& weight_packed, const at::Tensor& weight_scale,
@@ -263,20 +283,29 @@ std::tuple<at::Tensor, at::Tensor> repack_w4a16_gptq_cuda(const at::Tensor& qwei
     auto weight_marlin = at::empty({pw4_marlin_words(N, K)}, qw.options());
     at::Tensor perm = at::empty({0}, qw.options());
     const int32_t* pp = nullptr;
+    at::Tensor status;
+    StreamPoint sorted;
     if (g_idx.has_value() && g_idx->defined()) {
         TORCH_CHECK(g_idx->is_cuda() && g_idx->dim() == 1 && g_idx->size(0) == K,
                     "repack_w4a16_gptq: g_idx must be a CUDA [K] tensor");
         auto gi = g_idx->to(at::kInt).contiguous();
         perm = at::empty({K}, qw.options());
-        auto status = at::empty({1}, qw.options());
-        int rc = pw4_gidx_to_perm(gi.data_ptr<int32_t>(), K, group_size, perm.data_ptr<int32_t>(),
-                                  status.data_ptr<int32_t>(), current_stream());
+        // The status word lies in pinned host memory, which the kernel writes itself, and
+        // is read behind an event, after the repack is queued (its clamped reads are safe on
+        // any permutation): no copy back, and the device does not wait for the host.
+        status = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        const int rc = pw4_gidx_to_perm(gi.data_ptr<int32_t>(), K, group_size, perm.data_ptr<int32_t>(),
+                                        status.data_ptr<int32_t>(), current_stream());
         check_status(rc, "repack_w4a16_gptq");
-        TORCH_CHECK(status.item<int32_t>() == 0, "repack_w4a16_gptq: ", pw4_status_string(PW4_ERR_GIDX));
+        sorted.record(reinterpret_cast<hipStream_t>(current_stream()));
         pp = perm.data_ptr<int32_t>();
     }
     const int rc = pw4_repack_gptq(qw.data_ptr<int32_t>(), pp, N, K, weight_marlin.data_ptr<int32_t>(),
                                    current_stream());
+    if (status.defined()) {
+        sorted.wait();
+        TORCH_CHECK(*status.data_ptr<int32_t>() == 0, "repack_w4a16_gptq: ", pw4_status_string(PW4_ERR_GIDX));
+    }
     check_status(rc, "repack_w4a16_gptq");
     return {weight_marlin, perm};
 }

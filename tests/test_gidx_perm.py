@@ -1,0 +1,50 @@
+"""The act-order permutation at the edges of its variants: spans of one batch held in registers
+(K up to 4096, and 16384 with 16-byte loads), the two-walk spans past them, and the status from
+the counting workgroup (up to 16384 groups) or from the groups' own (past that)."""
+
+import numpy as np
+import pytest
+import torch
+
+from pulsar_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+# (K, G): K = 262160 has 16385 groups
+SIZES = [(16, 16), (4096, 16), (4112, 16), (16384, 128), (16512, 128), (262144, 16), (262160, 16)]
+
+
+def _g_idx(k, g, seed):
+    return np.random.default_rng(seed).permutation(np.arange(k, dtype=np.int32) // g)
+
+
+def _perm(g_idx, g, offset):
+    k = len(g_idx)
+    buf = torch.empty(k + offset, dtype=torch.int32, device="cuda")
+    buf[offset:].copy_(torch.from_numpy(g_idx))
+    qw = torch.zeros(k // 8, 8, dtype=torch.int32, device="cuda")
+    return ops.repack_w4a16_gptq(qw, buf[offset:], g)[1]
+
+
+@pytest.mark.parametrize("offset", [0, 1])  # 1: not 16-byte aligned
+@pytest.mark.parametrize("k,g", SIZES)
+def test_perm_is_the_stable_argsort(k, g, offset):
+    gi = _g_idx(k, g, k + offset)
+    want = np.argsort(gi, kind="stable").astype(np.int32)
+    for _ in range(2):
+        assert np.array_equal(_perm(gi, g, offset).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("k,g", SIZES)
+def test_bad_groupings_are_refused(k, g, offset):
+    ngroups = k // g
+    gi = _g_idx(k, g, k)
+    for at, value in ((0, -1), (k - 1, ngroups), (k // 2, (int(gi[k // 2]) + 1) % ngroups)):
+        bad = gi.copy()
+        bad[at] = value
+        if np.array_equal(bad, gi):  # a single group cannot be moved to another
+            continue
+        with pytest.raises(RuntimeError, match="g_idx"):
+            _perm(bad, g, offset)
+    assert np.array_equal(_perm(gi, g, offset).cpu().numpy(), np.argsort(gi, kind="stable"))
