@@ -338,35 +338,45 @@ struct KwavePlan {
     double us = 0.0;
 };
 
-// The cost model, fitted to graph periods of every (rows, columns, slices) plan
-// on the Llama-3-8B and -70B layers at M = 16..512 on one MI355X (within 10% of
-// the measured period on most of 420 plans):
-//   * a workgroup takes steps * c + e, with steps the 64-K chunks of its busiest
-//     wave and (c, e) by row tiles, 32-column tiles and dtype below (bf16's
-//     exact dequant takes twice the instructions); one workgroup runs per CU;
+// The cost model, fitted to graph periods of (rows, columns, slices) plans on the
+// Llama-3-8B and -70B layers and 4160 x 5000 at M = 16..1024 on one MI355X (the
+// picks take 1.6% longer than the best plan of each of 120 shapes):
+//   * one workgroup runs per CU and takes steps * c + e, with steps the 64-K chunks
+//     of its busiest wave and (c, e) by row tiles, 32-column tiles and dtype below
+//     (bf16's exact dequant takes twice the instructions); every round of
+//     workgroups past the first pays 2.5 us of its own start and drain, and 3% of all
+//     (the rounds drift apart: 70B o at M = 768, three rounds, 121 us against 113 on
+//     prefill tiles);
 //   * the weights, x and y stream at 5.2 TB/s; the two overlap, as the cube root
 //     of the sum of their cubes;
-//   * 4 us of launch, prologue and drain; K slices add 3.5 us and 0.25 per slice
-//     (device-scope partials, the last arriver's reads).
+//   * 4 us of launch, prologue and drain; K slices add 0.3 us, 0.35 per slice and
+//     their partial tiles' round trip at 4 TB/s.
+// Of equal plans the widest tile: its x is read by fewer workgroups (qkv M = 128
+// 14.4 us at 64 columns, 16.1 at 48).
 KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_t max_splits) {
-    constexpr double kStep[2][2][3] = {{{0.52, 0.76, 1.33}, {0.85, 1.17, 1.93}},
-                                       {{0.62, 1.00, 1.85}, {0.90, 1.30, 2.45}}};
+    constexpr double kStep[2][2][3] = {{{0.57, 0.76, 1.28}, {0.85, 1.15, 1.87}},
+                                       {{0.66, 1.00, 1.80}, {0.90, 1.28, 2.40}}};
     constexpr double kEnd[2][3] = {{0.6, 0.8, 1.5}, {0.8, 1.4, 2.6}};
     const double hbm = ((double)N * K * 0.515 + 2.0 * M * (N + K)) / 5.2e6;
     const int64_t nch = K / 64;
     KwavePlan best;
     for (int rt : {1, 2}) {
-        for (int nb : {16, 32, 48, 64, 96, 112, 128}) {
+        for (int nb : {128, 112, 96, 64, 48, 32, 16}) {
             const int ci = nb <= 32 ? 0 : nb <= 64 ? 1 : 2;
             const int64_t tiles = ceil_div(M, 32 * rt) * ceil_div(N, nb);
             for (int64_t s : {1, 2, 3, 4, 6, 8}) {
                 if (s > max_splits || (s > 1 && s * 8 > nch)) break;
                 const int64_t cps = ceil_div(nch, s);
                 if (s > 1 && ceil_div(nch, cps) != s) continue;  // the same plan as a smaller s
+                const double rounds = (double)ceil_div(tiles * s, (int64_t)cus);
                 const double cu =
-                    (double)ceil_div(tiles * s, (int64_t)cus) *
-                    ((double)ceil_div(cps, 8) * kStep[bf16][rt - 1][ci] + kEnd[rt - 1][ci]);
-                const double us = 4.0 + std::cbrt(hbm * hbm * hbm + cu * cu * cu) + (s > 1 ? 3.5 + 0.25 * (double)s : 0.0);
+                    (rounds * ((double)ceil_div(cps, 8) * kStep[bf16][rt - 1][ci] + kEnd[rt - 1][ci]) + 2.5 * (rounds - 1)) *
+                    (1.0 + 0.03 * (rounds - 1));
+                double us = 4.0 + std::cbrt(hbm * hbm * hbm + cu * cu * cu);
+                if (s > 1) {
+                    us += 0.3 + 0.35 * (double)s +
+                          (double)(tiles * s) * 4.0 * (double)kwave_tile_floats(rt, kwave_col_tiles(nb)) * 2.0 / 4e6;
+                }
                 if (best.nb == 0 || us < best.us) best = {rt, nb, s, us};
             }
         }
@@ -376,17 +386,27 @@ KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_
 
 // What the kernels beside it take, for the choice between them.  The prefill
 // model reads 4 us or more low (launch, ramp and, on K slices, the combine's).
-// The decode kernel at M = 17..32 streams the weights at about 2.5 TB/s behind
-// 4.5 us, and slows down with M (Llama-3-8B, us, decode / K-wave at M = 24 and
-// 32: qkv 10.7 / 9.0 and 11.4 / 9.6, o 7.7 / 8.1 and 9.0 / 8.4, gate_up 26.6 /
-// 18.9 and 29.0 / 19.9, down 22.8 / 14.3 and 24.3 / 14.9).
 double prefill_us(int64_t M, int64_t N, int64_t nchunks, int cus, bool only128) {
     double us = 0.0;
     plan_prefill256(M, N, nchunks, cus, only128, 8, &us);
     return us + 4.0;
 }
-double decode_m32_us(int64_t M, int64_t N, int64_t K) {
-    return (4.5 + (double)N * K / 2.0 / 2.5e6) * (0.7 + 0.0125 * (double)M);
+// The decode kernel: 4.6 us and the weights at 5 TB/s up to M = 16; past it two
+// 16-row tiles per wave, slower with the size of the layer and with M; 2 us for
+// each level of the exchange tree where x (M * K * 2 bytes) needs K slices to fit
+// in LDS (past M = 16, 0.3 for the first); half as much again for groups below 128,
+// whose MFMAs are masked.
+// Graph periods, us, fp16 x, decode / K-wave: qkv M = 17 10.6 / 8.2, M = 32 11.6 /
+// 9.4; o M = 17 7.7 / 7.8, M = 24 8.0 / 8.0, M = 32 9.0 / 8.3; gate_up M = 16 16.0 /
+// 18.2, M = 17 26.6 / 18.3; down M = 16 13.3 / 13.8, M = 17 17.3 / 13.8; 70B down M =
+// 32 67 / 32; 4160 x 5000 at G = 64 M = 8 9.6 / 8.5, M = 32 18.1 / 9.7.
+double decode_us(int64_t M, int64_t N, int64_t K, int64_t G) {
+    const double mb = (double)N * K / 2e6;
+    const int64_t slices = ceil_div(M * K * 2, 150000);
+    int levels = 0;
+    while ((int64_t{1} << levels) < slices) ++levels;
+    const double f = M <= 16 ? 1.0 : 1.0 + std::min(mb / 30.0, 0.55) + 0.01 * (double)(M - 17);
+    return (4.6 + mb / 5.0) * f * (G < 128 ? 1.5 : 1.0) + 2.0 * levels - (M > 16 && levels > 0 ? 1.7 : 0.0);
 }
 
 // K slices whose partial tiles stay within a workspace of ws_cap bytes (0: any).
@@ -397,8 +417,9 @@ int64_t max_kwave_splits(int64_t M, int64_t N, int64_t K, size_t ws_cap) {
     return fixed >= ws_cap ? 1 : std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)((ws_cap - fixed) / slice)));
 }
 
-// Decode batches up to this stay on the decode kernel.
-constexpr int64_t kKwaveMinM = 16;
+// Batches up to this stay on the decode kernel: half or more of a 32-row tile would be
+// padding, which its copies and MFMAs pay for.
+constexpr int64_t kKwaveMinM = 8;
 
 struct Plan {
     bool decode = false;
@@ -818,14 +839,21 @@ Plan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, i
     if (!kwave_override(&kp.rt, &kp.nb, &kp.splits, &never)) {
         if (never || plan_pinned()) return p;
         const double other_us = M <= 32 && (G & (G - 1)) == 0
-                                    ? decode_m32_us(M, N, K)
+                                    ? decode_us(M, N, K, G)
                                     : prefill_us(M, N, nch, cus, xt == X_F16 && prefill_exact_enabled());
+        // Only what looks clearly faster moves: the models are good to a few percent, and
+        // read low where the tiles take several rounds (o at M = 1024, two rounds: 47.2 us
+        // against a model of 44, prefill tiles 45.9).
+        auto faster = [&](const KwavePlan& k) {
+            const int64_t wgs = ceil_div(M, 32 * k.rt) * ceil_div(N, k.nb) * k.splits;
+            return k.us < (wgs <= cus ? 0.97 : 0.85) * other_us;
+        };
         kp = plan_kwave(M, N, K, xt == X_BF16, cus, max_kwave_splits(M, N, K, ws_cap));
-        if (kp.splits > 1 && kp.us < other_us &&
+        if (kp.splits > 1 && faster(kp) &&
             make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, 0, silu, ws_cap).workspace() == 0) {
             kp = plan_kwave(M, N, K, xt == X_BF16, cus, 1);
         }
-        if (kp.us >= other_us) return p;
+        if (!faster(kp)) return p;
     }
     const int64_t tiles = ceil_div(M, 32 * kp.rt) * ceil_div(N, kp.nb);
     if (kp.splits > 1 && tiles > kMaxCounterCols) return p;
@@ -845,9 +873,12 @@ Plan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, i
 
 // The same with the calling thread's last plans kept (by sizes alone): the
 // search takes about 2 us of host time, and one operator call plans three times.
+bool kwave_takes(int layout, int64_t M, int64_t N, int64_t K, int64_t G, int64_t num_splits) {
+    return M > kKwaveMinM && num_splits < 1 && (layout == LAYOUT_MARLIN || M > 32) && kwave_ok(N, K, G, 4);
+}
 Plan make_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
                      bool has_perm, int64_t num_splits, bool silu, size_t ws_cap) {
-    if (num_splits >= 1 || M <= kKwaveMinM || (layout != LAYOUT_MARLIN && M <= 32) || !kwave_ok(N, K, G, 4)) return {};
+    if (!kwave_takes(layout, M, N, K, G, num_splits)) return {};
     const int cus = cu_count();
     if (plan_overrides()) {  // they may change from call to call
         return search_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, silu, ws_cap, cus);
@@ -872,9 +903,10 @@ Plan make_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int
 // Workspace bytes of a call: for whichever of its two plans runs.
 size_t call_workspace(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
                       bool has_perm, int64_t num_splits, bool silu = false, size_t ws_cap = 0) {
+    const size_t base = make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, num_splits, silu, ws_cap).workspace();
+    if (!kwave_takes(layout, M, N, K, G, num_splits)) return base;
     return std::max(
-        make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, num_splits, silu, ws_cap).workspace(),
-        make_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, num_splits, silu, ws_cap).workspace());
+        base, make_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, num_splits, silu, ws_cap).workspace());
 }
 
 int check_common(int64_t M, int64_t N, int64_t K, int64_t G, int x_dtype) {
@@ -896,8 +928,11 @@ int run_gemm(int layout, const void* x, int x_dtype, const uint32_t* w, const vo
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) return PW4_ERR_ARG;
     // the medium-M kernel copies the scales as 4-byte words and needs its own scratch;
     // without either the call runs on its decode or prefill plan
-    Plan p = make_kwave_plan(layout, x_dtype, stype, qzeros != nullptr, M, N, K, G, perm != nullptr, num_splits, silu,
-                             ws_cap);
+    Plan p;
+    if (kwave_takes(layout, M, N, K, G, num_splits)) {
+        p = make_kwave_plan(layout, x_dtype, stype, qzeros != nullptr, M, N, K, G, perm != nullptr, num_splits, silu,
+                            ws_cap);
+    }
     if (!p.kwave || (layout == LAYOUT_MARLIN && (reinterpret_cast<uintptr_t>(scales) & 3) != 0) ||
         (p.workspace() > 0 && (workspace == nullptr || ws_bytes < p.workspace()))) {
         p = make_plan(layout, x_dtype, stype, qzeros != nullptr, M, N, K, G, perm != nullptr, num_splits, silu, ws_cap);

@@ -238,8 +238,9 @@ void kwave_kernel(const KwaveArgs a) {
     asm volatile("v_mov_b32 %0, %1" : "=v"(k64) : "s"(0x54005400u));
 
     // ---- one chunk --------------------------------------------------------------
-    auto step = [&](int j, auto st) {
+    auto step = [&](int j, auto st, auto refills) {
         constexpr int I = decltype(st)::value;
+        constexpr bool kRefills = decltype(refills)::value;
         const uint8_t* xa = xs(st) + wave * kStage;
         const uint8_t* sa = ss(st) + wave * kScaleSlot;
         u32x4 av[4][RT];
@@ -266,7 +267,8 @@ void kwave_kernel(const KwaveArgs a) {
         // the stage is in registers (the reads have returned), so its refill may go out
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
         __builtin_amdgcn_sched_barrier(0);
-        const Refill rf = prepare_refill(j + D);
+        Refill rf{};
+        if constexpr (kRefills) rf = prepare_refill(j + D);
 
         // scales: a column whose scale is zero in this group takes u = z and keeps its running scale
         bool tiny = false;
@@ -336,7 +338,8 @@ void kwave_kernel(const KwaveArgs a) {
                 const u32x4 bv = dequant(s, ct);
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) acc[rt][ct] = mfma32x32x16<BF16>(av[s][rt], bv, acc[rt][ct]);
-                if constexpr (s < 3) {
+                if constexpr (!kRefills) {
+                } else if constexpr (s < 3) {
                     copies(rf, Int<kCopies * i / (3 * C)>{}, Int<kCopies * (i + 1) / (3 * C)>{}, st);
                 } else {
                     load_w(rf, ct, st);
@@ -355,18 +358,28 @@ void kwave_kernel(const KwaveArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         },
         std::make_integer_sequence<int, D>{});
+    // Waves w and w + 4 share a SIMD: one of them goes ahead where both could issue, so that
+    // they do not run their dequant and their MFMAs in step (1-3% over the sizes above).
+    if (wave >= kWaves / 2) __builtin_amdgcn_s_setprio(2);
     const int nw_chunks = [&] {
         // chunks of this wave: whole rounds of eight runs, then its part of the last round
         const int n = max(c1 - c0, 0), round = 8 << rl;
         const int full = n / round, rest = n - full * round;
         return (full << rl) + min(max(rest - (wave << rl), 0), 1 << rl);
     }();
-    // Whole rounds of the ring: chunks past the wave's last are out of range, read as
-    // zeros from nowhere and add zero.  (Leaving in mid-round, or skipping their
-    // arithmetic, merges ring states, and the waits after it drain the ring.)
-    for (int j = 0; j < nw_chunks; j += D) {
-        unroll_seq([&](auto st) { step(j + decltype(st)::value, st); }, std::make_integer_sequence<int, D>{});
+    // Whole rounds of the ring (refills past the wave's last chunk are out of range: from
+    // nowhere), then the last chunks without refills.  Leaving a round in the middle, or
+    // skipping a refill, would merge ring states, and the waits after it drain the ring.
+    int j = 0;
+    for (; j + D <= nw_chunks; j += D) {
+        unroll_seq([&](auto st) { step(j + decltype(st)::value, st, std::true_type{}); },
+                   std::make_integer_sequence<int, D>{});
     }
+    unroll_seq(
+        [&](auto st) {
+            if (j + decltype(st)::value < nw_chunks) step(j + decltype(st)::value, st, std::false_type{});
+        },
+        std::make_integer_sequence<int, D - 1>{});
 
     // ---- sum of the waves in LDS, over the freed stages ----------------------------
     // A wave's accumulators are 16-byte quads (four rows of a column),
@@ -402,6 +415,7 @@ void kwave_kernel(const KwaveArgs a) {
                     *reinterpret_cast<f32x4*>(to + (((rt * C + ct) * 4 + e4) * 64 + lane) * 16) = v;
                 }
     };
+    __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_s_waitcnt(0);  // this wave's copies into LDS are done (those past its chunks too)
     __syncthreads();
     if constexpr (kTwoPhase) {

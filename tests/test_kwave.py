@@ -141,7 +141,7 @@ def test_default_plan_and_unaligned_scales(pin, m, n, k, g, dtype):
 @pytest.mark.parametrize("m,k,n,kwave", [
     # us on MI355X, graph periods, fp16 x: K-wave / the decode or prefill plan
     (24, 4096, 6144, True),    # 9.0 / 10.7
-    (24, 4096, 4096, False),   # 8.1 / 7.7
+    (17, 4096, 4096, False),   # 7.8 / 7.7
     (32, 4096, 28672, True),   # 19.9 / 29.0
     (32, 14336, 4096, True),   # 14.9 / 24.3
     (64, 4096, 4096, True),    # 9.2 / 19.0
@@ -150,6 +150,8 @@ def test_default_plan_and_unaligned_scales(pin, m, n, k, g, dtype):
     (256, 4096, 28672, False),  # 85 / 65.6
     (4096, 4096, 28672, False),
     (16, 4096, 28672, False),  # 18.2 / 16.0
+    (17, 4096, 28672, True),   # 18.3 / 26.6
+    (8, 4096, 4096, False),
 ])
 def test_planner(pin, m, k, n, kwave):
     pin(None)
