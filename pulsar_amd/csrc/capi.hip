@@ -715,7 +715,13 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
                 if (ncols % w != 0 || ceil_div(kps, 128) * w > 16 * 128) continue;
                 int64_t cost_w = 0;
                 const int64_t wps_w = pick_wps(ceil_div(ncols, w), &cost_w);
-                if (4 * wps_w < 3 * (int64_t)cus || 20 * cost_w * w > 23 * best_cost * 16) continue;
+                // (CT units get no more columns: a step of theirs reads 64-byte pieces of
+                // its columns, and fewer K waves read fewer of a line's pieces together.
+                // gate_up M = 1 18.1 us at 16 columns, 19.5 at 32, 22.2 at 64; qkv 7.5 / 7.2.)
+                if (4 * wps_w < 3 * (int64_t)cus ||
+                    20 * cost_w * w > (layout == LAYOUT_MARLIN ? 23 : 20) * best_cost * 16) {
+                    continue;
+                }
                 nb = w;
                 ncg = ceil_div(ncols, nb);
                 best_wps = wps_w;

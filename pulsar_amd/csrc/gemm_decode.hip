@@ -365,14 +365,17 @@ __global__ __launch_bounds__(WIN ? kThreads + 64 * kCopyWaves : kThreads) void d
             const uint32_t* seg = a.w + ((int64_t)(col0 >> 6) * a.nchunks + kc) * kChunkWords + (col0 & 63) * 4;
             o.w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(seg + (kc + 1 < a.nchunks ? lane_w : lane_w_tail)));
         } else {
+            // One range-checked 16-byte load whatever K: where K % 32 != 0 a row's last
+            // tile runs on into the next row (past the weights: zeros), against
+            // activations that are zero.  A branch for those rows, as this once had, made
+            // the compiler drain the ring before every load: gate_up M = 1 25.2 us.
             const int t = min(k0 / 32 + h, a.ktiles - 1);
-            const int64_t off = (int64_t)ncol_c * (K / 8) + t * 4;
-            if ((K & 31) == 0) {
-                o.w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.w + off));
-            } else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) o.w[q] = (t * 32 + q * 8 < K) ? a.w[off + q] : 0u;
-            }
+            const int64_t row_bytes = K / 2, unit_bytes = (int64_t)min(N - col0, nb) * row_bytes;
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+                (void*)(a.w + (int64_t)col0 * (K / 8)), (short)0,
+                (int)(uint32_t)min(unit_bytes, (int64_t)0xfffffff0), 0x00020000);
+            o.w = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)((uint32_t)(ncol_c - col0) * (uint32_t)row_bytes + t * 16),
+                                                        0, 2);  // (2: non-temporal)
         }
         if constexpr (SB) {
             if (head) {
@@ -423,11 +426,7 @@ __global__ __launch_bounds__(WIN ? kThreads + 64 * kCopyWaves : kThreads) void d
     }
 
     // ---- finish the slice: zero fill, (bf16) corrections ---------------------
-    if constexpr (LAYOUT == LAYOUT_MARLIN) {
-        wait_vmcnt<kRingLoads>();  // this wave's slice copies are done; its ring is still in flight
-    } else {
-        wait_vmcnt<0>();
-    }
+    wait_vmcnt<kRingLoads>();  // this wave's slice copies are done; its ring is still in flight
     if constexpr (PX) {
         // every wave's XN copies have landed (each waited for its own above);
         // slot (row, s8) of X gathers XN[row][perm[8 s8 .. 8 s8 + 7]]
