@@ -848,11 +848,11 @@ Plan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, i
                                     ? decode_us(M, N, K, G)
                                     : prefill_us(M, N, nch, cus, xt == X_F16 && prefill_exact_enabled());
         // Only what looks clearly faster moves: the models are good to a few percent, and
-        // read low where the tiles take several rounds (o at M = 1024, two rounds: 47.2 us
-        // against a model of 44, prefill tiles 45.9).
+        // against prefill tiles they read low where this kernel's take several rounds (o
+        // at M = 1024, two rounds: 47.2 us against a model of 44, prefill tiles 45.9).
         auto faster = [&](const KwavePlan& k) {
             const int64_t wgs = ceil_div(M, 32 * k.rt) * ceil_div(N, k.nb) * k.splits;
-            return k.us < (wgs <= cus ? 0.97 : 0.85) * other_us;
+            return k.us < (wgs <= cus || M <= 32 ? 0.97 : 0.85) * other_us;
         };
         kp = plan_kwave(M, N, K, xt == X_BF16, cus, max_kwave_splits(M, N, K, ws_cap));
         if (kp.splits > 1 && faster(kp) &&

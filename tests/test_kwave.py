@@ -151,6 +151,8 @@ def test_default_plan_and_unaligned_scales(pin, m, n, k, g, dtype):
     (4096, 4096, 28672, False),
     (16, 4096, 28672, False),  # 18.2 / 16.0
     (17, 4096, 28672, True),   # 18.3 / 26.6
+    (20, 8192, 57344, True),   # 54.5 / 91.7, two rounds of tiles
+    (1024, 4096, 4096, False),  # 47.2 / 45.9, two rounds of tiles
     (8, 4096, 4096, False),
 ])
 def test_planner(pin, m, k, n, kwave):
