@@ -471,6 +471,7 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
     // and 145 / 36, 70B gate_up 218 and 852 / 114, down 210 and 1031 / 74).
     bool decode_ok = M <= 32 && G >= 16 && (G & (G - 1)) == 0;
     const int decode_mode = decode_mode_override();
+    if (decode_mode == 0) decode_ok = false;
     const int xt = x_dtype == PW4_DTYPE_BF16 ? X_BF16 : X_F16;
     if (decode_ok && decode_mode != 1 && !forced && layout == LAYOUT_MARLIN &&
         prefer_prefill_tile(xt, M, N, K, G, cus)) {

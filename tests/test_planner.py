@@ -66,6 +66,13 @@ def test_70b_large_layers_decode_to_m28(lib, layer, m):
     assert plan(lib, m, k, n).startswith("decode"), plan(lib, m, k, n)
 
 
+@pytest.mark.parametrize("layout", [LAYOUT_CT, LAYOUT_MARLIN])
+@pytest.mark.parametrize("m", [1, 16, 32])
+def test_decode_override_zero_keeps_every_m_on_prefill(lib, monkeypatch, m, layout):
+    monkeypatch.setenv("PW4_DECODE", "0")
+    assert plan(lib, m, 4096, 4096, layout=layout).startswith("prefill")
+
+
 @pytest.mark.parametrize("layer", ["8b_qkv", "8b_o", "8b_gate_up", "8b_down", "70b_qkv"])
 @pytest.mark.parametrize("m", [1, 16, 28, 32])
 def test_other_layers_decode_up_to_m32(lib, layer, m):
