@@ -438,14 +438,14 @@ __global__ __launch_bounds__(kPermThreads) void repack_gptq_perm_kernel(const ui
 // loads its entries of kGidxBatch steps at once: the walks are bound by their
 // memory round trips.  ONE: a wave's span is one batch, whose matches stay in
 // registers, so pass 2 has no round trip of its own (K = 14336: 10.6 -> 6.9 us).
-// With one workgroup more than there are groups (hist_groups != 0), the last one
-// counts all groups in LDS and stores the status, so that no kernel has to clear
-// it first; else the groups' workgroups OR their findings into a cleared status.
+// One workgroup past the groups' counts all groups in LDS (kHistGroups at a time)
+// and stores the status, so that no kernel has to clear it first, and status may lie
+// in host memory, which atomics from the device need not reach.
+constexpr int kHistGroups = 16384;
 template <bool VEC, int kGidxWaves, int kGidxBatch, bool ONE>
 __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_t* __restrict__ g_idx,
                                                                     int32_t* __restrict__ perm,
-                                                                    int32_t* __restrict__ status, int K, int G,
-                                                                    int hist_groups) {
+                                                                    int32_t* __restrict__ status, int K, int G) {
     constexpr int EPL = VEC ? 4 : 1, kStep = 64 * EPL;
     static_assert(kGidxBatch * EPL <= 32, "a batch's matches are one word per lane");
     extern __shared__ int hist[];
@@ -473,28 +473,32 @@ __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_
         }
     };
     if (g == Kg) {  // the counting workgroup
-        for (int i = tid; i < Kg; i += 64 * kGidxWaves) hist[i] = 0;
         if (tid == 0) wave_cnt[0] = 0;
-        __syncthreads();
-        bool bad_id = false;
-        for (int k0 = k_begin; k0 < k_end; k0 += kStep * kGidxBatch) {
-            int gv[kGidxBatch][EPL];
-            load(k0, gv);
+        int st = 0;
+        for (int r = 0; r <= (Kg - 1) / kHistGroups; ++r) {
+            const int g0 = r * kHistGroups;
+            const int ng = min(Kg - g0, kHistGroups);
+            for (int i = tid; i < ng; i += 64 * kGidxWaves) hist[i] = 0;
+            __syncthreads();
+            for (int k0 = k_begin; k0 < k_end; k0 += kStep * kGidxBatch) {
+                int gv[kGidxBatch][EPL];
+                load(k0, gv);
 #pragma unroll
-            for (int b = 0; b < kGidxBatch; ++b)
+                for (int b = 0; b < kGidxBatch; ++b)
 #pragma unroll
-                for (int j = 0; j < EPL; ++j) {
-                    if (k0 + b * kStep + lane * EPL + j >= k_end) continue;
-                    if (gv[b][j] < 0 || gv[b][j] >= Kg) {
-                        bad_id = true;
-                    } else {
-                        atomicAdd(&hist[gv[b][j]], 1);
+                    for (int j = 0; j < EPL; ++j) {
+                        if (k0 + b * kStep + lane * EPL + j >= k_end) continue;
+                        if (gv[b][j] < 0 || gv[b][j] >= Kg) {
+                            st |= 2;
+                        } else if (gv[b][j] >= g0 && gv[b][j] - g0 < ng) {
+                            atomicAdd(&hist[gv[b][j] - g0], 1);
+                        }
                     }
-                }
+            }
+            __syncthreads();
+            for (int i = tid; i < ng; i += 64 * kGidxWaves) st |= hist[i] != G ? 1 : 0;
+            __syncthreads();
         }
-        __syncthreads();
-        int st = bad_id ? 2 : 0;
-        for (int i = tid; i < Kg; i += 64 * kGidxWaves) st |= hist[i] != G ? 1 : 0;
         if (st) atomicOr(&wave_cnt[0], st);
         __syncthreads();
         if (tid == 0) *status = wave_cnt[0];
@@ -510,7 +514,6 @@ __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_
 #pragma unroll
             for (int j = 0; j < EPL; ++j) {
                 const int k = k0 + b * kStep + lane * EPL + j;
-                if (hist_groups == 0 && g == 0 && k < k_end && (gv[b][j] < 0 || gv[b][j] >= Kg)) atomicOr(status, 2);
                 mine |= (uint32_t)(k < k_end && gv[b][j] == g) << (b * EPL + j);
             }
         return mine;
@@ -525,11 +528,10 @@ __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_
     }
     if (lane == 0) wave_cnt[wave] = count;
     __syncthreads();
-    int pos = 0, total = 0;
+    int pos = 0;
 #pragma unroll
     for (int w = 0; w < kGidxWaves; ++w) {
         pos += w < wave ? wave_cnt[w] : 0;
-        total += wave_cnt[w];
     }
     for (int k0 = k_begin; k0 < k_end; k0 += kStep * kGidxBatch) {
         const uint32_t mine = ONE ? first : batch(k0);
@@ -552,7 +554,6 @@ __global__ __launch_bounds__(64 * kGidxWaves) void gidx_perm_kernel(const int32_
             pos += step;
         }
     }
-    if (hist_groups == 0 && tid == 0 && total != G) atomicOr(status, 1);
 }
 
 __global__ __launch_bounds__(64) void clear_status_kernel(int32_t* __restrict__ status) {
@@ -677,21 +678,19 @@ hipError_t launch_repack_gptq(const uint32_t* qweight, const int32_t* perm, uint
 
 
 hipError_t launch_gidx_perm(const int32_t* g_idx, int32_t* perm, int32_t* status, int K, int G, hipStream_t stream) {
-    const int groups = K > 0 ? K / G : 0;
-    // The status from a counting workgroup beside the groups' where its counters fit
-    // in LDS, in place of a launch that clears it first (1.5 us and a gap).
-    const int hist = groups > 0 && groups <= 16384 ? groups : 0;
-    if (hist == 0) {
+    if (K == 0) {
         // cleared by a kernel rather than a memset, so that a caller capturing the
         // stream into a graph records a kernel node
         hipLaunchKernelGGL(clear_status_kernel, dim3(1), dim3(64), 0, stream, status);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess || K == 0) return e;
+        return hipGetLastError();
     }
-    const dim3 grid(groups + (hist ? 1 : 0));
-    const size_t lds = (size_t)hist * 4;
+    // The status comes from a counting workgroup beside the groups', in place of a launch
+    // that clears it first (1.5 us and a gap).
+    const int groups = K / G;
+    const dim3 grid(groups + 1);
+    const size_t lds = (size_t)std::min(groups, kHistGroups) * 4;
     auto go = [&](auto fn, int threads) {
-        hipLaunchKernelGGL(fn, grid, dim3(threads), lds, stream, g_idx, perm, status, K, G, hist);
+        hipLaunchKernelGGL(fn, grid, dim3(threads), lds, stream, g_idx, perm, status, K, G);
     };
     // Past K = 4096, eight waves with 16-byte loads where g_idx is 16-byte aligned
     // and K holds whole 4-entry runs (K = 14336: 17.4 -> 9.6 us, 28672: 29.2 ->

@@ -1,6 +1,6 @@
 """The act-order permutation at the edges of its variants: spans of one batch held in registers
 (K up to 4096, and 16384 with 16-byte loads), the two-walk spans past them, and the status from
-the counting workgroup (up to 16384 groups) or from the groups' own (past that)."""
+the counting workgroup, which takes 16384 groups at a time."""
 
 import numpy as np
 import pytest
@@ -40,7 +40,8 @@ def test_perm_is_the_stable_argsort(k, g, offset):
 def test_bad_groupings_are_refused(k, g, offset):
     ngroups = k // g
     gi = _g_idx(k, g, k)
-    for at, value in ((0, -1), (k - 1, ngroups), (k // 2, (int(gi[k // 2]) + 1) % ngroups)):
+    for at, value in ((0, -1), (k - 1, ngroups), (k // 2, (int(gi[k // 2]) + 1) % ngroups),
+                      (0, ngroups - 1 if gi[0] != ngroups - 1 else 0)):
         bad = gi.copy()
         bad[at] = value
         if np.array_equal(bad, gi):  # a single group cannot be moved to another
