@@ -27,6 +27,13 @@
 // multiplied by s_(g-1) / s_g when group g starts and by the last group's scale
 // at the end (a group whose scale is zero adds zero and is skipped).
 //
+// Range.  The running sum is y / s_g, which fp32 does not hold for every input that
+// y fits: scales far apart or (bf16) very large x overflow it.  A workgroup whose sums
+// come out infinite or NaN computes its slice again, each chunk's products scaled by
+// themselves, and a scale out of range (scale_in_range) makes them NaN.  fp16 x cannot get
+// there within that range, so fp16 x with fp16 scales has no check; the others look behind
+// their stores.
+//
 // K slices across workgroups (small N): every workgroup writes its fp32 tile
 // and the last to arrive for a tile (arrival counter) sums the slices in slice
 // order, stores y and resets the counter.
@@ -63,8 +70,13 @@ constexpr int kThreads = kKwaveThreads;
 static_assert(kThreads == kWaves * 64, "launch_kwave's block");
 constexpr int kScaleSlot = 768;  // per wave and stage: 512 bytes of scales, 256 of zero-point words
 
-// Scales below this magnitude count as zero: their reciprocal would overflow.
-constexpr float kTinyScale = 0x1p-120f;
+// Scales the running sum takes: 2^-41 <= |s| < 2^23 (infinities and NaN make their sums so
+// by themselves).  Two of them are less than 2^64 apart, so with fp16 x (2^16, times 15,
+// over K <= 2^22) it stays below 2^106.  Written so that its constants are inline ones:
+// the loop has no register for others.
+__device__ __forceinline__ bool scale_in_range(float s) {
+    return (uint32_t)(__builtin_amdgcn_frexp_expf(s) + 40) < 64u;
+}
 
 // Ring depth in chunks: LDS stages of x (RT * 4 KB per wave each, 128 KB in all)
 // and register sets of weight words.
@@ -97,7 +109,7 @@ void kwave_kernel(const KwaveArgs a) {
     __shared__ __attribute__((aligned(256))) uint8_t ss1[kWaves * kScaleSlot];
     __shared__ __attribute__((aligned(256))) uint8_t ss2[D > 2 ? kWaves * kScaleSlot : 16];
     __shared__ __attribute__((aligned(256))) uint8_t ss3[D > 2 ? kWaves * kScaleSlot : 16];
-    __shared__ int s_last;
+    __shared__ int s_bad, s_last;
     auto xs = [&](auto i) -> uint8_t* {
         constexpr int I = decltype(i)::value;
         if constexpr (I == 0) return xs0;
@@ -271,13 +283,13 @@ void kwave_kernel(const KwaveArgs a) {
         if constexpr (kRefills) rf = prepare_refill(j + D);
 
         // scales: a column whose scale is zero in this group takes u = z and keeps its running scale
-        bool tiny = false;
+        bool zero = false;
 #pragma unroll
-        for (int ct = 0; ct < C; ++ct) tiny |= __builtin_fabsf(sf[ct]) < kTinyScale;
-        if (__builtin_expect(__ballot(tiny) != 0, 0)) {
+        for (int ct = 0; ct < C; ++ct) zero |= sf[ct] == 0.f;
+        if (__builtin_expect(__ballot(zero) != 0, 0)) {
 #pragma unroll
             for (int ct = 0; ct < C; ++ct) {
-                const bool t = __builtin_fabsf(sf[ct]) < kTinyScale;
+                const bool t = sf[ct] == 0.f;
                 sf[ct] = t ? s_run[ct] : sf[ct];
                 const uint32_t zz = zw[ct] * 0x11111111u;
 #pragma unroll
@@ -289,7 +301,9 @@ void kwave_kernel(const KwaveArgs a) {
         if (kc < c1 && (j == 0 || group_of(kc) != group_of(chunk_at(j - 1)))) {
 #pragma unroll
             for (int ct = 0; ct < C; ++ct) {
-                const float r = s_run[ct] * __builtin_amdgcn_rcpf(sf[ct]);
+                float r = s_run[ct] * __builtin_amdgcn_rcpf(sf[ct]);
+                // (NaN sums are what the end of the slice looks for)
+                if constexpr (sizeof(ST) == 4) r = scale_in_range(sf[ct]) ? r : __builtin_bit_cast(float, 0xffffffffu);
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -381,15 +395,69 @@ void kwave_kernel(const KwaveArgs a) {
         },
         std::make_integer_sequence<int, D - 1>{});
 
+    // ---- the slice once more, each chunk's products scaled by themselves -------------
+    // (B of bf16 x is (u - z) / 1024, still exact, so that a chunk's sum is no larger than
+    // its largest x; plain loads: no measured workload comes here).  It takes its arguments
+    // and its lane index anew, or the compiler holds what it derives from them in registers
+    // through the whole slice: bf16 x, fp32 scales, zero points, gate_up M = 64 30.6 -> 33.1 us.
+    auto rescan = [&]() {
+        const KwaveArgs* p = reinterpret_cast<const KwaveArgs*>(
+            (const void*)__builtin_amdgcn_kernarg_segment_ptr());
+        asm volatile("" : "+s"(p));
+        int ln = threadIdx.x;
+        asm volatile("" : "+v"(ln));
+        const int c = ln & 31, h = (ln >> 5) & 1, wave = __builtin_amdgcn_readfirstlane(ln >> 6);
+        const int64_t N = p->N, K = p->K;
+        constexpr float kDown = BF16 ? 0x1p-10f : 1.f, kUp = 1.f / kDown;
+#pragma unroll
+        for (int ct = 0; ct < C; ++ct) {
+            s_run[ct] = 1.f;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[rt][ct][e] = 0.f;
+        }
+        const int end = min((split + 1) * p->chunks_per_split, p->nchunks);
+#pragma unroll 1
+        for (int kc = split * p->chunks_per_split + wave; kc < end; kc += kWaves) {
+            const int64_t g = kc / p->cpg;
+#pragma unroll
+            for (int ct = 0; ct < C; ++ct) {
+                const int n = min(n0 + ct * 32 + c, (int)N - 1);
+                const float s = (float)reinterpret_cast<const ST*>(p->scales)[g * N + n];
+                uint32_t z = 8u;
+                if constexpr (ZP) z = (p->qzeros[g * (N >> 3) + (n >> 3)] >> (4 * (n & 7))) & 0xfu;
+                const u32x4 q = *reinterpret_cast<const u32x4*>(
+                    p->w + ((int64_t)(n >> 6) * p->nchunks + kc) * kChunkWords + h * 256 + (n & 63) * 4);
+                auto weight = [&](uint32_t u) { return ((float)(u & 0xfu) - (float)z) * kDown; };
+                u32x4 bv[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int tg = 0; tg < 4; ++tg) {
+                        const uint32_t lo = f32_to_out<BF16>(weight(q[tg] >> (4 * i)));
+                        const uint32_t hi = f32_to_out<BF16>(weight(q[tg] >> (16 + 4 * i)));
+                        bv[i][tg] = lo | hi << 16;
+                    }
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const uint16_t* xr = p->x + min(m0 + rt * 32 + c, p->M - 1) * K + kc * 64 + h * 32;
+                    f32x16 t;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) t[e] = 0.f;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        t = mfma32x32x16<BF16>(*reinterpret_cast<const u32x4*>(xr + 8 * i), bv[i], t);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[rt][ct][e] += t[e] * s * kUp;
+                }
+            }
+        }
+    };
+
     // ---- sum of the waves in LDS, over the freed stages ----------------------------
     // A wave's accumulators are 16-byte quads (four rows of a column),
     // [tile][e / 4][lane]; quad q of the tile is summed by thread q % 512.
-#pragma unroll
-    for (int ct = 0; ct < C; ++ct)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[rt][ct][e] *= s_run[ct];
     constexpr int kTileBytes = RT * C * 4096;           // of one wave
     constexpr int kArray = kWaves * kStage;             // of one LDS variable
     constexpr bool kTwoPhase = kTileBytes * kWaves > kArray * D;
@@ -417,44 +485,54 @@ void kwave_kernel(const KwaveArgs a) {
     };
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_s_waitcnt(0);  // this wave's copies into LDS are done (those past its chunks too)
-    __syncthreads();
-    if constexpr (kTwoPhase) {
-        if (wave >= kParts) put(region(wave - kParts));
-        __syncthreads();
-        if (wave < kParts) {
-            const uint8_t* from = region(wave);
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int ct = 0; ct < C; ++ct)
-#pragma unroll
-                    for (int e4 = 0; e4 < 4; ++e4) {
-                        const f32x4 v =
-                            *reinterpret_cast<const f32x4*>(from + (((rt * C + ct) * 4 + e4) * 64 + lane) * 16);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[rt][ct][4 * e4 + e] += v[e];
-                    }
-        }
-        // (a wave overwrites only the region it read)
-        if (wave < kParts) put(region(wave));
-    } else {
-        put(region(wave));
-    }
-    __syncthreads();
+    if (tid == 0) s_bad = 0;
     constexpr int kQuads = RT * C * 256;
     constexpr int QT = (kQuads + kThreads - 1) / kThreads;  // quads per thread
     f32x4 sum[QT];
+    auto add_waves = [&]() {
 #pragma unroll
-    for (int i = 0; i < QT; ++i) {
-        const int q = tid + i * kThreads;
-        if (kQuads % kThreads != 0 && q >= kQuads) break;
-        f32x4 v[kParts];
+        for (int ct = 0; ct < C; ++ct)
 #pragma unroll
-        for (int w = 0; w < kParts; ++w) v[w] = *reinterpret_cast<const f32x4*>(region(w) + q * 16);
-        sum[i] = v[0];
+            for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int w = 1; w < kParts; ++w) sum[i] += v[w];
-    }
+                for (int e = 0; e < 16; ++e) acc[rt][ct][e] *= s_run[ct];
+        __syncthreads();
+        if constexpr (kTwoPhase) {
+            if (wave >= kParts) put(region(wave - kParts));
+            __syncthreads();
+            if (wave < kParts) {
+                const uint8_t* from = region(wave);
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+                        for (int e4 = 0; e4 < 4; ++e4) {
+                            const f32x4 v =
+                                *reinterpret_cast<const f32x4*>(from + (((rt * C + ct) * 4 + e4) * 64 + lane) * 16);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[rt][ct][4 * e4 + e] += v[e];
+                        }
+            }
+            // (a wave overwrites only the region it read)
+            if (wave < kParts) put(region(wave));
+        } else {
+            put(region(wave));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < QT; ++i) {
+            const int q = tid + i * kThreads;
+            if (kQuads % kThreads != 0 && q >= kQuads) break;
+            f32x4 v[kParts];
+#pragma unroll
+            for (int w = 0; w < kParts; ++w) v[w] = *reinterpret_cast<const f32x4*>(region(w) + q * 16);
+            sum[i] = v[0];
+#pragma unroll
+            for (int w = 1; w < kParts; ++w) sum[i] += v[w];
+        }
+    };
+    add_waves();
 
     // ---- output -----------------------------------------------------------------------
     auto store = [&](int q, const f32x4& v) {
@@ -486,12 +564,35 @@ void kwave_kernel(const KwaveArgs a) {
                 }
         }
     };
-    if (a.partial == nullptr) {
+    auto store_sums = [&]() {
 #pragma unroll
         for (int i = 0; i < QT; ++i) {
             const int q = tid + i * kThreads;
             if (kQuads % kThreads != 0 && q >= kQuads) break;
             store(q, sum[i]);
+        }
+    };
+    constexpr bool kCheck = BF16 || sizeof(ST) == 4;  // (see Range)
+    auto look = [&]() {
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < QT; ++i) {
+            if (kQuads % kThreads != 0 && tid + i * kThreads >= kQuads) break;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bad |= !(__builtin_fabsf(sum[i][e]) <= 0x1.fffffep127f);
+        }
+        if (__ballot(bad) != 0 && lane == 0) s_bad = 1;
+    };
+    if (a.partial == nullptr) {
+        store_sums();
+        if constexpr (kCheck) {
+            look();
+            __syncthreads();  // (and every wave has read the regions)
+            if (__builtin_expect(s_bad, 0)) {
+                rescan();
+                add_waves();
+                store_sums();
+            }
         }
         return;
     }
@@ -501,20 +602,31 @@ void kwave_kernel(const KwaveArgs a) {
     auto part = [&](int sp, int q) {
         return reinterpret_cast<uint64_t*>(a.partial + (((int64_t)tile * a.splits + sp) * kQuads + q) * 4);
     };
+    auto write_part = [&]() {
 #pragma unroll
-    for (int i = 0; i < QT; ++i) {
-        const int q = tid + i * kThreads;
-        if (kQuads % kThreads != 0 && q >= kQuads) break;
-        uint64_t* p = part(split, q);
+        for (int i = 0; i < QT; ++i) {
+            const int q = tid + i * kThreads;
+            if (kQuads % kThreads != 0 && q >= kQuads) break;
+            uint64_t* p = part(split, q);
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const uint64_t v = (uint64_t)__builtin_bit_cast(uint32_t, (float)sum[i][2 * e]) |
-                               ((uint64_t)__builtin_bit_cast(uint32_t, (float)sum[i][2 * e + 1]) << 32);
-            __hip_atomic_store(p + e, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int e = 0; e < 2; ++e) {
+                const uint64_t v = (uint64_t)__builtin_bit_cast(uint32_t, (float)sum[i][2 * e]) |
+                                   ((uint64_t)__builtin_bit_cast(uint32_t, (float)sum[i][2 * e + 1]) << 32);
+                __hip_atomic_store(p + e, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if constexpr (kCheck) look();
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+    };
+    write_part();
+    if constexpr (kCheck) {
+        if (__builtin_expect(s_bad, 0)) {
+            rescan();
+            add_waves();
+            write_part();
         }
     }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
     if (tid == 0) {
         s_last = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
                  a.splits - 1;
@@ -548,12 +660,7 @@ void kwave_kernel(const KwaveArgs a) {
                 }
         }
     }
-#pragma unroll
-    for (int i = 0; i < QT; ++i) {
-        const int q = tid + i * kThreads;
-        if (kQuads % kThreads != 0 && q >= kQuads) break;
-        store(q, sum[i]);
-    }
+    store_sums();
     if (tid == 0) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #endif
 }

@@ -106,6 +106,60 @@ def test_zero_and_negative_scales(pin, plan, dtype):
     assert (y[:, 3] == 0).all()
 
 
+def _ref64(c, g):
+    """x @ dequant(W)^T in 64 bits, for scales and activations whose fp32 sums could overflow."""
+    w = (c.u.astype(np.float64) - c.z.T.repeat(g, axis=1)) * np.repeat(c.scale_nk.astype(np.float64), g, axis=1)
+    return c.x.double().cpu().numpy() @ w.T
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sym", [True, False])
+@pytest.mark.parametrize("low", [2.0 ** -40, 2.0 ** -45, 2.0 ** -119, 1e-40, 2.0 ** 45])
+@pytest.mark.parametrize("plan", ["1,64,1", "2,128,2", "1,128,3", "2,32,1"])
+def test_scales_far_from_their_neighbours(pin, plan, low, sym, dtype):
+    """A group whose scale is many powers of two below (or above) the others': the sum behind it,
+    in its units, is past fp32, but y is not."""
+    if low > 1 and dtype == torch.float16:
+        pytest.skip("activations of 2^-45 are not fp16 values")
+    m, n, k, g = 40, 256, 2048, 128
+    c = baseline_case(m, n, k, g, dtype=dtype, seed=11, symmetric=sym)
+    s = np.full_like(c.scale_nk, 16.0)
+    s[:, 5] = low
+    s[7, 1:] = low      # all groups but the first, or the last
+    s[9, :-1] = low
+    s[11] = low         # every group
+    s[13, 3:] = 0.0
+    c.scale_nk = s.astype(np.float32)
+    if low > 1:  # y of ordinary size again
+        c.x = (c.x.float() * 2.0 ** -45).to(dtype)
+    ref = _ref64(c, g)
+    pin(plan)
+    y = _run(c, g, torch.float32, False, sym)
+    cols = [i for i in range(n) if i not in (11, 7, 9)] if low > 1 else list(range(n))
+    check(y[:, cols], ref[:, cols], dtype, f"{plan} low={low} {dtype}", abs_excess=False)
+    for i in (7, 9, 11):  # against their own size: their sums may be far from the others'
+        r = ref[:, i]
+        if np.abs(r).max() > 1e-37 and dtype == torch.bfloat16 or np.abs(r).max() > 1e-2:
+            assert np.abs(y[:, i].double().cpu().numpy() - r).max() <= 2e-2 * np.abs(r).max(), (i, low)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sdtype,sym", [(torch.float16, True), (torch.float32, False)])
+@pytest.mark.parametrize("plan", ["1,64,1", "2,128,2"])
+def test_large_bf16_activations(pin, plan, sdtype, sym):
+    """Activations near bf16's largest, scaled by a power of two: the same result, scaled."""
+    m, n, k, g = 40, 256, 2048, 128
+    c = baseline_case(m, n, k, g, dtype=torch.bfloat16, seed=12, symmetric=sym)
+    pin(plan)
+    y = _run(c, g, sdtype, False, sym)
+    check(y, c.y_ref, torch.bfloat16, plan)
+    c.x = (c.x.float() * 2.0 ** 121).to(torch.bfloat16)
+    assert c.x.isfinite().all()
+    scaled = _run(c, g, sdtype, False, sym).double() * 2.0 ** -121
+    check(scaled, c.y_ref, torch.bfloat16, plan + " scaled")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_infinite_and_nan_rows_stay_in_their_rows(pin, dtype):
