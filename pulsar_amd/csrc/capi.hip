@@ -832,19 +832,17 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
     return p;
 }
 
-// The medium-M kernel's plan of a call (kwave false where another kernel is the
-// faster one, or the call is not one it takes).  The CT layout reaches it past
-// the decode range only, repacked; forced K splits and pinned plans never.  A call
-// whose decode or prefill plan needs no workspace takes no K slices here either.
-Plan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
-                       bool has_perm, bool silu, size_t ws_cap, int cus) {
-    Plan p;
+// The medium-M kernel's tile and K slices for a call (nb 0 where another kernel is the
+// faster one).  Pinned plans never take it.  A call whose decode or prefill plan needs
+// no workspace takes no K slices here either.
+KwavePlan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
+                            bool has_perm, bool silu, size_t ws_cap, int cus) {
     const int xt = x_dtype == PW4_DTYPE_BF16 ? X_BF16 : X_F16;
     const int64_t nch = K / 64;
     KwavePlan kp;
     bool never = false;
     if (!kwave_override(&kp.rt, &kp.nb, &kp.splits, &never)) {
-        if (never || plan_pinned()) return p;
+        if (never || plan_pinned()) return {};
         const double other_us = M <= 32 && (G & (G - 1)) == 0
                                     ? decode_us(M, N, K, G)
                                     : prefill_us(M, N, nch, cus, xt == X_F16 && prefill_exact_enabled());
@@ -860,10 +858,78 @@ Plan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, i
             make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, 0, silu, ws_cap).workspace() == 0) {
             kp = plan_kwave(M, N, K, xt == X_BF16, cus, 1);
         }
-        if (!faster(kp)) return p;
+        if (!faster(kp)) return {};
     }
-    const int64_t tiles = ceil_div(M, 32 * kp.rt) * ceil_div(N, kp.nb);
-    if (kp.splits > 1 && tiles > kMaxCounterCols) return p;
+    if (kp.splits > 1 && ceil_div(M, 32 * kp.rt) * ceil_div(N, kp.nb) > kMaxCounterCols) return {};
+    return kp;
+}
+
+// The calls the kernel takes.  Forced K splits never; the CT layout past the decode
+// range only, repacked.
+bool kwave_takes(int layout, int64_t M, int64_t N, int64_t K, int64_t G, int64_t num_splits) {
+    return M > kKwaveMinM && num_splits < 1 && (layout == LAYOUT_MARLIN || M > 32) && kwave_ok(N, K, G, 4);
+}
+
+// The calling thread's last searches, by everything a search depends on: one takes about 3 us
+// of host time, and one operator call plans three times (the workspace of both activation
+// dtypes, then the run, whose scale type and zero points the workspace query does not know).
+// Sets of four, so that the few keys of a call, and of the layers that alternate with it,
+// do not evict each other: with one slot a set, and a set that did not tell scale types
+// apart, a call with symmetric weights searched twice each time (o at M = 9..64: 6.3 us for
+// a query and a plan, now 0.7-0.9).
+class KwavePlanTable {
+   public:
+    using Key = std::array<int64_t, 7>;
+    template <typename F>
+    const KwavePlan& get(const Key& key, F&& search) {
+        uint64_t h = 0;
+        for (int64_t v : key) {
+            h = (h ^ (uint64_t)v) * 0x9e3779b97f4a7c15ull;
+            h ^= h >> 32;
+        }
+        Set& set = sets_[h % kSets];
+        for (Entry& e : set.ways) {
+            if (e.key == key) return e.plan;
+        }
+        Entry& e = set.ways[set.next++ % kWays];
+        e.plan = search();
+        e.key = key;
+        return e.plan;
+    }
+
+   private:
+    static constexpr size_t kSets = 64, kWays = 4;
+    struct Entry {
+        Key key{-1};  // (no call has M = -1)
+        KwavePlan plan;
+    };
+    struct Set {
+        std::array<Entry, kWays> ways;
+        unsigned next = 0;
+    };
+    std::array<Set, kSets> sets_;
+};
+
+// The medium-M kernel's plan of a call (kwave false where it does not run on it).
+Plan make_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
+                     bool has_perm, int64_t num_splits, bool silu, size_t ws_cap) {
+    Plan p;
+    if (!kwave_takes(layout, M, N, K, G, num_splits)) return p;
+    const int cus = cu_count();
+    auto search = [&] {
+        return search_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, silu, ws_cap, cus);
+    };
+    KwavePlan kp;
+    if (plan_overrides()) {  // they may change from call to call
+        kp = search();
+    } else {
+        static thread_local KwavePlanTable table;
+        kp = table.get({M, N, K, G, (int64_t)ws_cap, cus,
+                        layout | x_dtype << 4 | stype << 8 | (int)zp << 12 | (int)has_perm << 13 | (int)silu << 14},
+                       search);
+    }
+    if (kp.nb == 0) return p;
+    const int64_t nch = K / 64;
     p.kwave = true;
     p.kw_rt = kp.rt;
     p.kw_nb = kp.nb;
@@ -871,40 +937,12 @@ Plan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, i
     p.splits = (int)ceil_div(nch, p.kw_cps);
     p.use_partial = p.splits > 1;
     if (p.use_partial) {
-        p.partial_bytes = (size_t)tiles * p.splits * kwave_tile_floats(kp.rt, kwave_col_tiles(kp.nb)) * 4;
+        p.partial_bytes = (size_t)(ceil_div(M, 32 * kp.rt) * ceil_div(N, kp.nb)) * p.splits *
+                          kwave_tile_floats(kp.rt, kwave_col_tiles(kp.nb)) * 4;
     }
     if (layout == LAYOUT_CT) p.repack_bytes = ct_repack_bytes(N, K, G);
     if (has_perm) p.xperm_bytes = (size_t)M * K * 2;
     return p;
-}
-
-// The same with the calling thread's last plans kept (by sizes alone): the
-// search takes about 2 us of host time, and one operator call plans three times.
-bool kwave_takes(int layout, int64_t M, int64_t N, int64_t K, int64_t G, int64_t num_splits) {
-    return M > kKwaveMinM && num_splits < 1 && (layout == LAYOUT_MARLIN || M > 32) && kwave_ok(N, K, G, 4);
-}
-Plan make_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N, int64_t K, int64_t G,
-                     bool has_perm, int64_t num_splits, bool silu, size_t ws_cap) {
-    if (!kwave_takes(layout, M, N, K, G, num_splits)) return {};
-    const int cus = cu_count();
-    if (plan_overrides()) {  // they may change from call to call
-        return search_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, silu, ws_cap, cus);
-    }
-    using Key = std::array<int64_t, 7>;
-    const Key key{M, N, K, G, (int64_t)ws_cap, cus,
-                  layout | x_dtype << 4 | stype << 8 | (int)zp << 12 | (int)has_perm << 13 | (int)silu << 14};
-    struct Entry {
-        Key key{-1};
-        Plan plan;
-    };
-    constexpr size_t kEntries = 64;
-    static thread_local Entry table[kEntries];
-    Entry& e = table[(size_t)(M * 31 + N / 8 * 7 + K / 64 * 3 + key[6]) % kEntries];
-    if (e.key != key) {
-        e.plan = search_kwave_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, silu, ws_cap, cus);
-        e.key = key;
-    }
-    return e.plan;
 }
 
 // Workspace bytes of a call: for whichever of its two plans runs.

@@ -1,0 +1,139 @@
+"""The table that keeps a thread's last medium-M plans.  It is by-passed where PW4_* overrides may
+change a plan from call to call, which tests/conftest.py enables, so everything here runs in a
+child process without them, as a user's program does."""
+
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes, itertools, json, sys, time
+sys.path[:0] = [%r, %r]
+import pulsar_amd
+from pw4_capi import DTYPE_BF16, DTYPE_F16, DTYPE_F32, declare
+lib = declare(pulsar_amd.capi())
+lib.pw4_medium_plan_describe.argtypes = [ctypes.c_int] * 6 + [ctypes.c_int64] * 5 + [ctypes.c_char_p, ctypes.c_size_t]
+buf = ctypes.create_string_buffer(160)
+def describe(layout, dtype, stype, zp, perm, silu, m, n, k, g=128):
+    assert lib.pw4_medium_plan_describe(layout, dtype, stype, zp, perm, silu, m, n, k, g, 0, buf, len(buf)) == 0
+    return buf.value.decode()
+""" % (ROOT, os.path.join(ROOT, "tests"))
+
+
+def _child(body, overrides, timeout=240):
+    env = {k: v for k, v in os.environ.items() if not k.startswith("PW4_")}
+    if overrides:
+        env["PW4_PLAN_OVERRIDES"] = "1"
+    r = subprocess.run([sys.executable, "-c", PRELUDE + body], env=env, capture_output=True, text=True,
+                       timeout=timeout)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+    return r.stdout.strip().splitlines()[-1]
+
+
+# more keys than the table has entries, each asked for again behind others
+PLANS = """
+cases = [(layout, dtype, stype, zp, perm, silu, m, n, k)
+         for m, (n, k) in itertools.product((9, 17, 32, 33, 64, 197, 512), ((4096, 4096), (28672, 4096), (4096, 14336),
+                                                                            (5008, 4224)))
+         for layout, dtype, stype, zp, perm, silu in itertools.product((0, 1), (DTYPE_F16, DTYPE_BF16),
+                                                                       (DTYPE_F16, DTYPE_F32), (0, 1), (0, 1), (0, 1))]
+out = [describe(*c) for c in cases]
+for step in (1, 7, 131):
+    assert [describe(*c) for c in cases[::step]] == out[::step]
+for a, b in zip(cases[::5], cases[3::11]):
+    assert (describe(*a), describe(*b), describe(*a)) == (out[cases.index(a)], out[cases.index(b)], out[cases.index(a)])
+print(json.dumps(out))
+"""
+
+
+def test_the_table_answers_what_a_search_does():
+    kept, searched = json.loads(_child(PLANS, False)), json.loads(_child(PLANS, True))
+    assert kept == searched
+    assert len(set(kept)) > 4
+
+
+# A workspace query plans for fp16 scales with zero points, the run for its own; neither may
+# push the other out.  The yardstick is the run whose key agrees with the query's.
+HOST_TIME = """
+def pair(stype, zp, silu, m, n, k):
+    query = lib.pw4_gemm_w4a16_silu_mul_workspace_size if silu else lib.pw4_gemm_w4a16_marlin_workspace_size
+    args = (m, n, k, 128, 0) if silu else (m, n, k, 128, 0, 0)
+    best = 1e9
+    for _ in range(15):
+        t = time.perf_counter()
+        for _ in range(100):
+            query(*args)
+            describe(1, DTYPE_F16, stype, zp, 0, silu, m, n, k)
+        best = min(best, (time.perf_counter() - t) / 100)
+    return best
+out = []
+for m, (n, k), silu in itertools.product((9, 16, 64), ((4096, 4096), (28672, 4096)), (0, 1)):
+    same = pair(DTYPE_F16, 1, silu, m, n, k)
+    for stype, zp in ((DTYPE_F16, 0), (DTYPE_F32, 0), (DTYPE_F32, 1)):
+        out.append((m, n, silu, stype, zp, pair(stype, zp, silu, m, n, k) / same))
+print(json.dumps(out))
+"""
+
+
+def test_a_query_and_its_run_keep_both_plans():
+    for m, n, silu, stype, zp, ratio in json.loads(_child(HOST_TIME, False)):
+        # a search of each costs 2 to 4 times the calls themselves, ctypes included
+        assert ratio < 1.6, (m, n, silu, stype, zp, ratio)
+
+
+# One shape through the workspace entry points and the no-alloc one (whose plans differ by its
+# scratch), alternating with others, dtypes, act-order and the SiLU gate.
+GPU_CALLS = """
+import numpy as np, torch
+from pulsar_amd import ops
+from w4a16_case import baseline_case, check
+from oracle import oracle as O
+G = 128
+def silu(y):
+    t = y.astype(np.float64).reshape(y.shape[0], -1, 2, 8)
+    return (t[:, :, 0] / (1 + np.exp(-t[:, :, 0])) * t[:, :, 1]).reshape(y.shape[0], -1)
+calls = []
+for m, n, k in ((33, 1024, 2048), (64, 512, 4096), (20, 1536, 4096)):
+    for dtype in (torch.float16, torch.bfloat16):
+        for sym, act in ((True, False), (False, True)):
+            c = baseline_case(m, n, k, G, dtype=dtype, seed=m + n, symmetric=sym, act_order=act)
+            wm, perm = ops.repack_w4a16_gptq(c.qweight(), torch.from_numpy(c.g_idx).cuda() if act else None, G)
+            for sdt in (torch.float16, torch.float32):
+                s = c.scale(sdt, kn=True)
+                calls.append((c, wm, s, None if sym else c.qzeros(), perm if act else None, dtype))
+def noalloc(c, wm, s, qz, perm, dtype):
+    y = torch.empty(c.m, c.n, dtype=dtype, device="cuda")
+    rc = lib.pw4_gemm_w4a16_marlin_noalloc(
+        c.x.data_ptr(), DTYPE_BF16 if dtype == torch.bfloat16 else DTYPE_F16, wm.data_ptr(), s.data_ptr(),
+        DTYPE_F32 if s.dtype == torch.float32 else DTYPE_F16, None if qz is None else qz.data_ptr(),
+        None if perm is None else perm.data_ptr(), y.data_ptr(), c.m, c.n, c.k, G, 0,
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, rc
+    return y
+plans = set()
+for _ in range(2):
+    for c, wm, s, qz, perm, dtype in calls:
+        what = "%s %s %s %s" % ((c.m, c.n, c.k), dtype, s.dtype, perm is not None)
+        print(what, flush=True)
+        plans.add(describe(1, DTYPE_BF16 if dtype == torch.bfloat16 else DTYPE_F16, DTYPE_F16, int(qz is not None),
+                           int(perm is not None), 0, c.m, c.n, c.k).split()[0])
+        y = ops.gemm_w4a16_gptq(c.x, wm, s, qz, perm, G)
+        check(y, c.y_ref, dtype, what)
+        check(noalloc(c, wm, s, qz, perm, dtype), c.y_ref, dtype, what + " no-alloc")
+        if s.dtype == torch.float16:
+            check(ops.gemm_w4a16_silu_mul(c.x, wm, s, qz, perm, G), silu(c.y_ref), dtype, what + " silu",
+                  abs_excess=False)
+        assert torch.equal(ops.gemm_w4a16_gptq(c.x, wm, s, qz, perm, G), y), what
+assert "kwave" in plans, plans
+print("done")
+"""
+
+
+@pytest.mark.gpu
+def test_calls_on_kept_plans_match_the_oracle():
+    assert _child(GPU_CALLS, False) == "done"
