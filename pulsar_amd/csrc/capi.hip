@@ -336,6 +336,12 @@ struct KwavePlan {
     int rt = 1, nb = 0;
     int64_t splits = 1;
     double us = 0.0;
+    // bytes of its K slices' partial tiles, whole tiles of 32-column tiles each
+    size_t partial_bytes(int64_t M, int64_t N) const {
+        if (splits <= 1) return 0;
+        return (size_t)(ceil_div(M, 32 * rt) * ceil_div(N, nb) * splits) *
+               (size_t)kwave_tile_floats(rt, kwave_col_tiles(nb)) * sizeof(float);
+    }
 };
 
 // The cost model, fitted to graph periods of (rows, columns, slices) plans on the
@@ -353,7 +359,8 @@ struct KwavePlan {
 //     their partial tiles' round trip at 4 TB/s.
 // Of equal plans the widest tile: its x is read by fewer workgroups (qkv M = 128
 // 14.4 us at 64 columns, 16.1 at 48).
-KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_t max_splits) {
+// max_partial: bytes the partial tiles may take.
+KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_t max_splits, size_t max_partial) {
     constexpr double kStep[2][2][3] = {{{0.57, 0.76, 1.28}, {0.85, 1.15, 1.87}},
                                        {{0.66, 1.00, 1.80}, {0.90, 1.28, 2.40}}};
     constexpr double kEnd[2][3] = {{0.6, 0.8, 1.5}, {0.8, 1.4, 2.6}};
@@ -368,6 +375,7 @@ KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_
                 if (s > max_splits || (s > 1 && s * 8 > nch)) break;
                 const int64_t cps = ceil_div(nch, s);
                 if (s > 1 && ceil_div(nch, cps) != s) continue;  // the same plan as a smaller s
+                if (KwavePlan{rt, nb, s}.partial_bytes(M, N) > max_partial) break;
                 const double rounds = (double)ceil_div(tiles * s, (int64_t)cus);
                 const double cu =
                     (rounds * ((double)ceil_div(cps, 8) * kStep[bf16][rt - 1][ci] + kEnd[rt - 1][ci]) + 2.5 * (rounds - 1)) *
@@ -407,14 +415,6 @@ double decode_us(int64_t M, int64_t N, int64_t K, int64_t G) {
     while ((int64_t{1} << levels) < slices) ++levels;
     const double f = M <= 16 ? 1.0 : 1.0 + std::min(mb / 30.0, 0.55) + 0.01 * (double)(M - 17);
     return (4.6 + mb / 5.0) * f * (G < 128 ? 1.5 : 1.0) + 2.0 * levels - (M > 16 && levels > 0 ? 1.7 : 0.0);
-}
-
-// K slices whose partial tiles stay within a workspace of ws_cap bytes (0: any).
-int64_t max_kwave_splits(int64_t M, int64_t N, int64_t K, size_t ws_cap) {
-    if (ws_cap == 0) return 8;
-    // a slice's partial tiles cover at most (M + 63) x (N + 127) outputs
-    const size_t slice = (size_t)(M + 63) * (N + 127) * 4, fixed = kZeroRegion + (size_t)M * K * 2 + 4 * kAlign;
-    return fixed >= ws_cap ? 1 : std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)((ws_cap - fixed) / slice)));
 }
 
 // Batches up to this stay on the decode kernel: half or more of a 32-row tile would be
@@ -839,6 +839,11 @@ KwavePlan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t
                             bool has_perm, bool silu, size_t ws_cap, int cus) {
     const int xt = x_dtype == PW4_DTYPE_BF16 ? X_BF16 : X_F16;
     const int64_t nch = K / 64;
+    // what a workspace of ws_cap bytes has left for partial tiles (beside x in the permuted
+    // order; a plan without them takes what the call's other plan takes, or less)
+    const size_t fixed = kZeroRegion + kAlign + (has_perm ? align_up((size_t)M * K * 2) : 0) +
+                         (layout == LAYOUT_CT ? align_up(ct_repack_bytes(N, K, G)) : 0);
+    const size_t max_partial = ws_cap == 0 ? SIZE_MAX : ws_cap > fixed ? ws_cap - fixed : 0;
     KwavePlan kp;
     bool never = false;
     if (!kwave_override(&kp.rt, &kp.nb, &kp.splits, &never)) {
@@ -853,14 +858,15 @@ KwavePlan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t
             const int64_t wgs = ceil_div(M, 32 * k.rt) * ceil_div(N, k.nb) * k.splits;
             return k.us < (wgs <= cus || M <= 32 ? 0.97 : 0.85) * other_us;
         };
-        kp = plan_kwave(M, N, K, xt == X_BF16, cus, max_kwave_splits(M, N, K, ws_cap));
+        kp = plan_kwave(M, N, K, xt == X_BF16, cus, 8, max_partial);
         if (kp.splits > 1 && faster(kp) &&
             make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, 0, silu, ws_cap).workspace() == 0) {
-            kp = plan_kwave(M, N, K, xt == X_BF16, cus, 1);
+            kp = plan_kwave(M, N, K, xt == X_BF16, cus, 1, 0);
         }
         if (!faster(kp)) return {};
     }
     if (kp.splits > 1 && ceil_div(M, 32 * kp.rt) * ceil_div(N, kp.nb) > kMaxCounterCols) return {};
+    if (kp.partial_bytes(M, N) > max_partial) return {};  // (a pinned plan)
     return kp;
 }
 
@@ -936,10 +942,7 @@ Plan make_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int
     p.kw_cps = (int)ceil_div(nch, std::min<int64_t>(kp.splits, nch));
     p.splits = (int)ceil_div(nch, p.kw_cps);
     p.use_partial = p.splits > 1;
-    if (p.use_partial) {
-        p.partial_bytes = (size_t)(ceil_div(M, 32 * kp.rt) * ceil_div(N, kp.nb)) * p.splits *
-                          kwave_tile_floats(kp.rt, kwave_col_tiles(kp.nb)) * 4;
-    }
+    p.partial_bytes = KwavePlan{kp.rt, kp.nb, p.splits}.partial_bytes(M, N);
     if (layout == LAYOUT_CT) p.repack_bytes = ct_repack_bytes(N, K, G);
     if (has_perm) p.xperm_bytes = (size_t)M * K * 2;
     return p;

@@ -17,7 +17,7 @@ import torch
 
 import pulsar_amd
 from pulsar_amd import ops
-from pw4_capi import DTYPE_BF16, DTYPE_F16
+from pw4_capi import DTYPE_BF16, DTYPE_F16, PW4_NOALLOC_SCRATCH_BYTES, declare
 from w4a16_case import baseline_case, check
 
 
@@ -190,6 +190,25 @@ def test_default_plan_and_unaligned_scales(pin, m, n, k, g, dtype):
     assert describe(m, k, n, g, DTYPE_BF16 if dtype == torch.bfloat16 else DTYPE_F16).startswith("kwave")
     for offset in (0, 1):
         check(_run(c, g, torch.float16, False, True, offset), c.y_ref, dtype, f"m={m} offset={offset}")
+
+
+@pytest.mark.gpu
+def test_no_alloc_call_whose_slices_do_not_fit_its_scratch(pin):
+    """16-column tiles take 32 columns of partial tile each: eight slices of 200 x 4096 need 59 MB
+    beside the 16 MB zero region, more than the no-alloc scratch.  The call runs its other plan."""
+    m, n, k, g = 200, 4096, 4096, 128
+    c = baseline_case(m, n, k, g, seed=21)
+    wm, _ = ops.repack_w4a16_gptq(c.qweight(), None, g)
+    s = c.scale(torch.float16, kn=True)
+    lib = declare(pulsar_amd.capi())
+    pin("1,16,8")
+    assert lib.pw4_gemm_w4a16_marlin_workspace_size(m, n, k, g, 0, 0) > PW4_NOALLOC_SCRATCH_BYTES
+    y = torch.empty(m, n, dtype=torch.float16, device="cuda")
+    rc = lib.pw4_gemm_w4a16_marlin_noalloc(c.x.data_ptr(), DTYPE_F16, wm.data_ptr(), s.data_ptr(), DTYPE_F16, None,
+                                           None, y.data_ptr(), m, n, k, g, 0,
+                                           torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, rc
+    check(y, c.y_ref, torch.float16, "no-alloc")
 
 
 @pytest.mark.parametrize("m,k,n,kwave", [
