@@ -104,7 +104,7 @@ int pw4_plan_describe(int layout, int x_dtype, int scale_dtype, int has_zp, int 
                       int64_t N, int64_t K, int64_t group_size, int64_t num_splits, char* buf, size_t len);
 
 /* The same for the medium-M kernel (MARLIN words, or CT words repacked per
- * call; K and the group size multiples of 64, N of 8): "kwave rows=64 nb=112
+ * call; K and the group size multiples of 64, N of 8): "kwave rows=64 nb=128
  * splits=1" (rows and columns of a tile, K slices) where the call runs on it,
  * else "none".  A call whose scales are not 4-byte aligned, or whose workspace
  * holds only its decode or prefill plan, runs on that plan. */

@@ -357,8 +357,10 @@ struct KwavePlan {
 //     of the sum of their cubes;
 //   * 4 us of launch, prologue and drain; K slices add 0.3 us, 0.35 per slice and
 //     their partial tiles' round trip at 4 TB/s.
-// Of equal plans the widest tile: its x is read by fewer workgroups (qkv M = 128
-// 14.4 us at 64 columns, 16.1 at 48).
+// The widths are those of the three kernels (4, 2 and 1 column tiles): a narrower tile runs
+// the next wider kernel, for the same time a chunk and no fewer workgroups, and its x is
+// read by more of them (qkv M = 128 14.4 us at 64 columns, 16.1 at 48).  Of equal plans
+// the widest.
 // max_partial: bytes the partial tiles may take.
 KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_t max_splits, size_t max_partial) {
     constexpr double kStep[2][2][3] = {{{0.57, 0.76, 1.28}, {0.85, 1.15, 1.87}},
@@ -368,7 +370,7 @@ KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_
     const int64_t nch = K / 64;
     KwavePlan best;
     for (int rt : {1, 2}) {
-        for (int nb : {128, 112, 96, 64, 48, 32, 16}) {
+        for (int nb : {128, 64, 32}) {
             const int ci = nb <= 32 ? 0 : nb <= 64 ? 1 : 2;
             const int64_t tiles = ceil_div(M, 32 * rt) * ceil_div(N, nb);
             for (int64_t s : {1, 2, 3, 4, 6, 8}) {
@@ -876,7 +878,7 @@ bool kwave_takes(int layout, int64_t M, int64_t N, int64_t K, int64_t G, int64_t
     return M > kKwaveMinM && num_splits < 1 && (layout == LAYOUT_MARLIN || M > 32) && kwave_ok(N, K, G, 4);
 }
 
-// The calling thread's last searches, by everything a search depends on: one takes about 3 us
+// The calling thread's last searches, by everything a search depends on: one takes about 2 us
 // of host time, and one operator call plans three times (the workspace of both activation
 // dtypes, then the run, whose scale type and zero points the workspace query does not know).
 // Sets of four, so that the few keys of a call, and of the layers that alternate with it,

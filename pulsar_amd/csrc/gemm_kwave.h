@@ -2,9 +2,9 @@
 // fp16 or bf16 activations, K and the group size multiples of 64.
 //
 // Work split.  A workgroup of eight waves owns a tile of up to 32 * RT rows by
-// nb <= 32 * C columns over one K slice; the waves split the slice's 64-K
-// chunks between them, and every wave computes the whole tile over its own
-// chunks.  So a weight word is loaded and dequantized by exactly one wave, an
+// nb <= 32 * C columns over one K slice (the planner gives whole column tiles, a
+// pinned plan any multiple of 16); the waves split the slice's 64-K chunks
+// between them, and every wave computes the whole tile over its own chunks.  So a weight word is loaded and dequantized by exactly one wave, an
 // activation fragment is read from LDS once and used for all C column tiles,
 // and no wave waits for another before the end: each has its own LDS ring of
 // activations and its own register ring of weight words.  The eight partial
