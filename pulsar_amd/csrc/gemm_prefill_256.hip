@@ -362,11 +362,10 @@ void prefill256_kernel(const PrefillArgs a, const NibbleMasks mk) {
         }
         return g;
     };
-    // Unsplit 128-row tiles run two workgroups per CU: one of them goes ahead where both
-    // could issue, so that they do not dequantize and multiply in step (gate_up M = 4096
-    // 837 -> 826 us, M = 1024 243 -> 236; K halves and 256-row tiles, whose waves share
-    // their barriers, were up to 7% slower with it).
-    if (RT == 4 && KS == 1 && ((blockIdx.x >> 8) & 1)) __builtin_amdgcn_s_setprio(2);
+    // (see launch_variant)
+    if (RT == 4 && KS == 1 && !PARTIAL && a.ahead != 0 && ((blockIdx.x / (unsigned)a.ahead) & 1)) {
+        __builtin_amdgcn_s_setprio(2);
+    }
     if (nck > 0) issue(c_begin, 0, next_group());
     if (nck > 1) issue(c_begin + 1, 1, next_group());
     int gk = EXACT ? c_begin % cpg : 0;  // place of the chunk being computed in its group
@@ -616,6 +615,16 @@ void launch_variant(const PrefillArgs& a, hipStream_t stream, KernelEvents ev) {
         return;
     }
     if (a.tile_rows == TM / 2) {  // every tile 128 rows: twice the workgroups, two per CU
+        // With a second round of pairs that is more than half full, every second run of `cus`
+        // workgroups (the later of a CU's two, in the first round) issues ahead: the pairs end,
+        // and begin their second round, at different times.  776 to 1024 workgroups on 256
+        // CUs, fp16 and bf16, both scale types: 1-6% faster from 16 chunks on (gate_up M =
+        // 1024 229 -> 221.5 us, 1408 x 20000 235 -> 225.6), at 8 chunks 5% faster to 3%
+        // slower.  Up to 768 workgroups it is within 1% either way; past 1024 it was 17%
+        // slower (1232 and 1280 workgroups at 8 chunks) to 4% faster (1344), and on K slices
+        // 7% slower (2048 x 6144 x 14336 on four), so those run without.
+        const int64_t cus = a.cus;
+        w.ahead = tiles128 > 3 * cus && tiles128 <= 4 * cus && a.nchunks >= 16 ? a.cus : 0;
         half(dim3((unsigned)tiles128), w, ev.start, ev.stop, std::false_type{});
         return;
     }

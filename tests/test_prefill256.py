@@ -105,6 +105,22 @@ def test_prefill_tail_split(plan_env):
     check(y, c.y_ref, torch.float16, "tail split m=1024 n=18432")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,k", [(3072, 1024), (3200, 1024), (3200, 960), (4096, 1024), (4224, 1024)])
+def test_prefill_second_round_of_pairs(plan_env, m, k, dtype):
+    """768, 800, 1024 and 1056 unsplit 128-row tiles: on 256 CUs both sides of the grids whose
+    second workgroup of each CU issues ahead, and 15 chunks, which do not.  Every fourth row
+    of each 128-row tile against the oracle."""
+    plan_env["PW4_PREFILL_ROWS"] = "128"
+    plan_env["PW4_PREFILL_SPLITS"] = "1"
+    n, g = 8192, 64
+    rows = np.arange(0, m, 4)
+    c = baseline_case(m, n, k, g, dtype=dtype, seed=m + k, rows=rows)
+    wm, _ = ops.repack_w4a16_gptq(c.qweight(), None, g)
+    y = ops.gemm_w4a16_gptq(c.x, wm, c.scale(torch.float16, kn=True), None, None, g)
+    check(y[torch.from_numpy(rows).cuda()], c.y_ref, dtype, f"m={m} k={k} {dtype}")
+
+
 @pytest.mark.parametrize("exact", ["1", "0"], ids=["exact", "rounded"])
 @pytest.mark.parametrize("rows", [256, 128])
 @pytest.mark.parametrize("splits", [1, 3, 8])
