@@ -104,10 +104,8 @@ class StreamPoint {
     ~StreamPoint() {
         if (ev_ != nullptr) (void)hipEventDestroy(ev_);
     }
-    void record(hipStream_t stream) {
-        check(hipEventCreateWithFlags(&ev_, hipEventDisableTiming));
-        check(hipEventRecord(ev_, stream));
-    }
+    void create() { check(hipEventCreateWithFlags(&ev_, hipEventDisableTiming)); }
+    void record(hipStream_t stream) { check(hipEventRecord(ev_, stream)); }
     void wait() { check(hipEventSynchronize(ev_)); }
 
    private:
@@ -288,6 +286,13 @@ std::tuple<at::Tensor, at::Tensor> repack_w4a16_gptq_cuda(const at::Tensor& qwei
     if (g_idx.has_value() && g_idx->defined()) {
         TORCH_CHECK(g_idx->is_cuda() && g_idx->dim() == 1 && g_idx->size(0) == K,
                     "repack_w4a16_gptq: g_idx must be a CUDA [K] tensor");
+        // The host waits below, which a capture has no place for; and a graph's replays would
+        // write the status long after its word is freed.  Refused before anything is recorded.
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        TORCH_CHECK(hipStreamIsCapturing(reinterpret_cast<hipStream_t>(current_stream()), &cs) == hipSuccess &&
+                        cs == hipStreamCaptureStatusNone,
+                    "repack_w4a16_gptq: an act-order repack cannot be captured into a graph");
+        sorted.create();
         auto gi = g_idx->to(at::kInt).contiguous();
         perm = at::empty({K}, qw.options());
         // The status word lies in pinned host memory, which the kernel writes itself, and

@@ -49,3 +49,26 @@ def test_bad_groupings_are_refused(k, g, offset):
         with pytest.raises(RuntimeError, match="g_idx"):
             _perm(bad, g, offset)
     assert np.array_equal(_perm(gi, g, offset).cpu().numpy(), np.argsort(gi, kind="stable"))
+
+
+def test_refused_under_capture():
+    """The host reads the status, so the call cannot be captured: it raises before it records
+    anything, and the capture around it stays whole."""
+    k, g = 4096, 128
+    gi = _g_idx(k, g, 3)
+    qw = torch.zeros(k // 8, 64, dtype=torch.int32, device="cuda")
+    t = torch.from_numpy(gi).cuda()
+    x = torch.arange(64, dtype=torch.float32, device="cuda")
+    ops.repack_w4a16_gptq(qw, t, g)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="captured"):
+            ops.repack_w4a16_gptq(qw, t, g)
+        y = x * 2
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, x * 2)
+    assert np.array_equal(_perm(gi, g, 0).cpu().numpy(), np.argsort(gi, kind="stable"))
