@@ -834,6 +834,26 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
     return p;
 }
 
+// The decode kernel's time from its plan, fitted to graph periods of 3000 calls of M = 9..32,
+// N = 256..57344, K = 256..28672, G = 64 and 128, both activation dtypes (half of them within
+// 6%): a launch, the copy of x, the busiest workgroup's units (an end, and 128-K steps of a K
+// wave, by M past 16 and G below 128) beside the weight stream, and the slices' exchange.
+// decode_us above is fitted on the layers of 8 MB and more, and reads up to twice the time
+// on smaller ones, above all in groups of 64, where the line would go wrong by itself:
+// 2048 x 2560 at M = 9, G = 64 4.4 us here against 6.1 on the medium-M kernel.
+double decode_plan_us(const Plan& p, bool bf16, int64_t M, int64_t N, int64_t K, int64_t G) {
+    constexpr double kStep[2][2] = {{0.243, 0.458}, {0.609, 0.882}};
+    const DecodeConfig& dc = p.dc;
+    const bool big = M > 16;
+    const double units = (double)ceil_div(ceil_div(round_up(N, kMarlinBN), dc.nb), dc.wps);
+    const double steps = (double)ceil_div(ceil_div(dc.k_per_split, 128) * (dc.nb / 16), 8);
+    const double step = kStep[big][G < 128] * (bf16 ? 1.117 : 1.0) * (1.0 + 0.022 * (double)(big ? M - 17 : 0));
+    const double cu = units * ((big ? 0.6 : 0.94) + steps * step);
+    const double hbm = (double)N * K * 0.515 / 4.6e6;
+    const double x = dc.kwin > 0 ? 0.0 : (double)M * dc.k_per_split * 1.16e-5;
+    return 2.2 + x + std::cbrt(cu * cu * cu + hbm * hbm * hbm) + 1.08 * std::log2((double)dc.splits);
+}
+
 // The medium-M kernel's tile and K slices for a call (nb 0 where another kernel is the
 // faster one).  Pinned plans never take it.  A call whose decode or prefill plan needs
 // no workspace takes no K slices here either.
@@ -850,19 +870,24 @@ KwavePlan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t
     bool never = false;
     if (!kwave_override(&kp.rt, &kp.nb, &kp.splits, &never)) {
         if (never || plan_pinned()) return {};
+        const Plan other = make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, 0, silu, ws_cap);
         const double other_us = M <= 32 && (G & (G - 1)) == 0
                                     ? decode_us(M, N, K, G)
                                     : prefill_us(M, N, nch, cus, xt == X_F16 && prefill_exact_enabled());
+        // (the price of a medium-M plan reads about 1 us high at these M; up to 24 MB of weights
+        // decode_plan_us is the closer one, past it decode_us is)
+        const double plan_us =
+            other.decode ? (N * K < (int64_t{48} << 20) ? 0.92 : 1.05) * decode_plan_us(other, xt == X_BF16, M, N, K, G) + 1.0
+                         : 1e30;
         // Only what looks clearly faster moves: the models are good to a few percent, and
         // against prefill tiles they read low where this kernel's take several rounds (o
         // at M = 1024, two rounds: 47.2 us against a model of 44, prefill tiles 45.9).
         auto faster = [&](const KwavePlan& k) {
             const int64_t wgs = ceil_div(M, 32 * k.rt) * ceil_div(N, k.nb) * k.splits;
-            return k.us < (wgs <= cus || M <= 32 ? 0.97 : 0.85) * other_us;
+            return k.us < (wgs <= cus || M <= 32 ? 0.97 : 0.85) * other_us && k.us < plan_us;
         };
         kp = plan_kwave(M, N, K, xt == X_BF16, cus, 8, max_partial);
-        if (kp.splits > 1 && faster(kp) &&
-            make_plan(layout, x_dtype, stype, zp, M, N, K, G, has_perm, 0, silu, ws_cap).workspace() == 0) {
+        if (kp.splits > 1 && faster(kp) && other.workspace() == 0) {
             kp = plan_kwave(M, N, K, xt == X_BF16, cus, 1, 0);
         }
         if (!faster(kp)) return {};

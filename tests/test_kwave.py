@@ -233,6 +233,22 @@ def test_planner(pin, m, k, n, kwave):
     assert (describe(m, k, n) != "none") == kwave, describe(m, k, n)
 
 
+@pytest.mark.parametrize("m,k,n,g,dtype,kwave", [
+    # the same on small layers, where a launch and the units' ends are most of the decode kernel's
+    # time: K-wave / decode
+    (9, 2048, 2560, 64, DTYPE_BF16, False),    # 6.1 / 4.4
+    (9, 3072, 4096, 64, DTYPE_F16, False),     # 6.7 / 5.0
+    (16, 512, 1024, 64, DTYPE_F16, False),     # 4.2 / 3.5
+    (32, 1024, 4096, 128, DTYPE_BF16, False),  # 5.3 / 4.3
+    (32, 1536, 2560, 64, DTYPE_BF16, False),   # 5.9 / 5.3
+    (9, 8192, 8192, 64, DTYPE_BF16, True),     # 14.3 / 16.7 (M = 10)
+    (13, 14336, 4096, 64, DTYPE_BF16, True),   # 14.3 / 16.4
+])
+def test_planner_on_small_layers(pin, m, k, n, g, dtype, kwave):
+    pin(None)
+    assert (describe(m, k, n, g, dtype) != "none") == kwave, describe(m, k, n, g, dtype)
+
+
 def test_planner_keeps_what_the_kernel_does_not_take(pin):
     pin(None)
     assert describe(64, 4096, 4096, splits=2) == "none"   # a forced K split
