@@ -361,6 +361,11 @@ struct KwavePlan {
 // the next wider kernel, for the same time a chunk and no fewer workgroups, and its x is
 // read by more of them (qkv M = 128 14.4 us at 64 columns, 16.1 at 48).  Of equal plans
 // the widest.
+// The price of the pick has a third part under that root, which the choice among plans
+// is better without: an XCD reads a row tile's x once for the column tiles that its
+// workgroups run side by side (tiles run down the rows first, an eighth of them on each
+// XCD), and the XCDs take 7.5 TB/s of it together.  With few columns and many rows it is
+// the longest: M = 2048, 12288 x 512 58 us, of which the steps are 29; 40 on prefill tiles.
 // max_partial: bytes the partial tiles may take.
 KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_t max_splits, size_t max_partial) {
     constexpr double kStep[2][2][3] = {{{0.57, 0.76, 1.28}, {0.85, 1.15, 1.87}},
@@ -369,6 +374,7 @@ KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_
     const double hbm = ((double)N * K * 0.515 + 2.0 * M * (N + K)) / 5.2e6;
     const int64_t nch = K / 64;
     KwavePlan best;
+    double cubes = 0.0;  // its steps' and stream's
     for (int rt : {1, 2}) {
         for (int nb : {128, 64, 32}) {
             const int ci = nb <= 32 ? 0 : nb <= 64 ? 1 : 2;
@@ -387,10 +393,17 @@ KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_
                     us += 0.3 + 0.35 * (double)s +
                           (double)(tiles * s) * 4.0 * (double)kwave_tile_floats(rt, kwave_col_tiles(nb)) * 2.0 / 4e6;
                 }
-                if (best.nb == 0 || us < best.us) best = {rt, nb, s, us};
+                if (best.nb == 0 || us < best.us) {
+                    best = {rt, nb, s, us};
+                    cubes = hbm * hbm * hbm + cu * cu * cu;
+                }
             }
         }
     }
+    const double rows = (double)ceil_div(M, 32 * best.rt), tiles = rows * (double)ceil_div(N, best.nb);
+    const double shared = std::max(1.0, std::floor(std::min(tiles, (double)cus) / 8.0 / rows));
+    const double xcd = tiles * 64.0 * best.rt * (double)K / shared / 7.5e6;
+    best.us += std::cbrt(cubes + xcd * xcd * xcd) - std::cbrt(cubes);
     return best;
 }
 

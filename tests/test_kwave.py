@@ -249,6 +249,20 @@ def test_planner_on_small_layers(pin, m, k, n, g, dtype, kwave):
     assert (describe(m, k, n, g, dtype) != "none") == kwave, describe(m, k, n, g, dtype)
 
 
+@pytest.mark.parametrize("m,k,n,dtype,kwave", [
+    # few columns and many rows, where every XCD reads all of x: K-wave / prefill tiles
+    (2048, 12288, 512, DTYPE_F16, False),   # 58.4 / 40.2
+    (4096, 8192, 128, DTYPE_BF16, False),   # 41.3 / 29.2
+    (1500, 8192, 512, DTYPE_F16, False),    # 34.6 / 27.7
+    (2048, 8192, 1024, DTYPE_F16, False),
+    (1024, 16384, 512, DTYPE_F16, False),   # 47.4 / 37.2
+    (2048, 4096, 1024, DTYPE_F16, True),    # 29.0 / 32.0
+])
+def test_planner_on_narrow_layers(pin, m, k, n, dtype, kwave):
+    pin(None)
+    assert (describe(m, k, n, 128, dtype) != "none") == kwave, describe(m, k, n, 128, dtype)
+
+
 def test_planner_keeps_what_the_kernel_does_not_take(pin):
     pin(None)
     assert describe(64, 4096, 4096, splits=2) == "none"   # a forced K split
