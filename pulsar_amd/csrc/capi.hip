@@ -847,24 +847,32 @@ Plan make_plan(int layout, int x_dtype, int stype, bool zp, int64_t M, int64_t N
     return p;
 }
 
-// The decode kernel's time from its plan, fitted to graph periods of 3000 calls of M = 9..32,
+// The decode kernel's time from its plan, fitted to graph periods of 3036 calls of M = 9..32,
 // N = 256..57344, K = 256..28672, G = 64 and 128, both activation dtypes (half of them within
-// 6%): a launch, the copy of x, the busiest workgroup's units (an end, and 128-K steps of a K
-// wave, by M past 16 and G below 128) beside the weight stream, and the slices' exchange.
-// decode_us above is fitted on the layers of 8 MB and more, and reads up to twice the time
-// on smaller ones, above all in groups of 64, where the line would go wrong by itself:
-// 2048 x 2560 at M = 9, G = 64 4.4 us here against 6.1 on the medium-M kernel.
-double decode_plan_us(const Plan& p, bool bf16, int64_t M, int64_t N, int64_t K, int64_t G) {
-    constexpr double kStep[2][2] = {{0.243, 0.458}, {0.609, 0.882}};
+// 4%, nine in ten within 10): a launch; the copy of x, by K windows the longer one; the
+// busiest workgroup's units (an end, by the unit's width, and 128-K steps of a K wave, by
+// M past 16 and G below 128; 3/4 more for each further workgroup of its CU) beside the weight
+// stream, as the root of the sum of their squares; the slices' exchange or partial tiles.
+// decode_us above is fitted on large layers, and reads up to twice the time on small ones,
+// above all in groups of 64, where the line would go wrong by it alone: 2048 x 2560 at M = 9,
+// G = 64 4.4 us here against 6.1 on the medium-M kernel.
+double decode_plan_us(const Plan& p, bool bf16, int64_t M, int64_t N, int64_t K, int64_t G, int cus) {
+    constexpr double kStep[2][2] = {{0.116, 0.298}, {0.287, 0.575}};
     const DecodeConfig& dc = p.dc;
-    const bool big = M > 16;
+    const bool big = M > 16, win = dc.kwin > 0;
+    const double slices = (double)dc.splits, width = (double)(dc.nb / 16);
     const double units = (double)ceil_div(ceil_div(round_up(N, kMarlinBN), dc.nb), dc.wps);
-    const double steps = (double)ceil_div(ceil_div(dc.k_per_split, 128) * (dc.nb / 16), 8);
-    const double step = kStep[big][G < 128] * (bf16 ? 1.117 : 1.0) * (1.0 + 0.022 * (double)(big ? M - 17 : 0));
-    const double cu = units * ((big ? 0.6 : 0.94) + steps * step);
-    const double hbm = (double)N * K * 0.515 / 4.6e6;
-    const double x = dc.kwin > 0 ? 0.0 : (double)M * dc.k_per_split * 1.16e-5;
-    return 2.2 + x + std::cbrt(cu * cu * cu + hbm * hbm * hbm) + 1.08 * std::log2((double)dc.splits);
+    // (waves that run one step fewer leave the others their share)
+    const double even = (double)(ceil_div(dc.k_per_split, 128) * (dc.nb / 16)) / 8.0;
+    const double steps = std::max(1.0, 0.5 * (even + std::ceil(even)));
+    const double step = kStep[big][G < 128] * (bf16 ? 1.2 : 1.0) * (big ? 1.0 + 0.01 * (double)(M - 17) : 1.0);
+    const double end = big ? 0.91 + 1.27 * (width - 1.0) : 1.0 + 1.15 * (width - 1.0);
+    const double resident = (double)ceil_div((int64_t)dc.wps * dc.splits, (int64_t)cus);
+    const double cu = units * (end + steps * step * (win ? 0.82 : 1.0)) * (1.0 + 0.76 * (resident - 1.0));
+    const double hbm = (double)N * K * 0.515 / 7e6;
+    const double x = win ? (double)M * K * 4.0e-5 : (double)M * dc.k_per_split * 2.45e-5;
+    const double sum = p.tree ? 0.94 * std::log2(slices) : p.use_partial ? 0.78 * slices : 0.0;
+    return 2.1 + x + std::sqrt(cu * cu + hbm * hbm) + sum;
 }
 
 // The medium-M kernel's tile and K slices for a call (nb 0 where another kernel is the
@@ -887,11 +895,9 @@ KwavePlan search_kwave_plan(int layout, int x_dtype, int stype, bool zp, int64_t
         const double other_us = M <= 32 && (G & (G - 1)) == 0
                                     ? decode_us(M, N, K, G)
                                     : prefill_us(M, N, nch, cus, xt == X_F16 && prefill_exact_enabled());
-        // (the price of a medium-M plan reads about 1 us high at these M; up to 24 MB of weights
-        // decode_plan_us is the closer one, past it decode_us is)
-        const double plan_us =
-            other.decode ? (N * K < (int64_t{48} << 20) ? 0.92 : 1.05) * decode_plan_us(other, xt == X_BF16, M, N, K, G) + 1.0
-                         : 1e30;
+        // (the price of a medium-M plan reads 1 us high at these M, past 8 us more than a tenth)
+        const double own_us = other.decode ? decode_plan_us(other, xt == X_BF16, M, N, K, G, cus) : 1e30;
+        const double plan_us = std::max(0.97 * own_us + 1.0, 1.1 * own_us);
         // Only what looks clearly faster moves: the models are good to a few percent, and
         // against prefill tiles they read low where this kernel's take several rounds (o
         // at M = 1024, two rounds: 47.2 us against a model of 44, prefill tiles 45.9).
