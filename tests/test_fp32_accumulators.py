@@ -19,6 +19,8 @@ Reference counterparts: the split paths behind gemm_w4a16_split / gemm_w4a16_mar
 north star's max-abs 1e-2.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -103,25 +105,49 @@ def test_pre_cast_accumulators(env, plan, m, n, k, slices, bf16, act):
     assert err <= MAX_ABS, f"{what}: accumulator max-abs {err:.3e} > {MAX_ABS}"
 
 
-# The default plans (no forced split), whose accumulators never reach memory:
-# pw4_observe_next_call arms the call to write the fp32 value each y element is
-# rounded from.  (name, M, N, K, bf16 x, act-order, workspace expected)
+# The unforced plans, whose accumulators never reach memory: pw4_observe_next_call
+# arms the call to write the fp32 value each y element is rounded from.
+# (name, PW4_KWAVE, M, N, K, bf16 x, act-order, workspace expected): "0" keeps the call off the
+# medium-M kernel, which by itself takes some of these sizes; the others pin its tile
 DEFAULT_PLAN_CASES = [
-    ("decode direct store", 4, 2048, 14336, False, False, False),
-    ("decode direct store, act-order", 8, 1024, 8192, False, True, False),
-    ("decode exchange tree", 16, 1024, 14336, False, False, True),
-    ("decode exchange tree, bf16", 32, 1024, 4096, True, False, True),
-    ("decode exchange tree, act-order", 16, 1024, 28672, False, True, True),
-    ("prefill unsplit, exact scaling", 4096, 4096, 14336, False, False, False),
-    ("prefill K slices + combine", 256, 4096, 14336, False, False, True),
+    ("decode direct store", "0", 4, 2048, 14336, False, False, False),
+    ("decode direct store, act-order", "0", 8, 1024, 8192, False, True, False),
+    ("decode exchange tree", "0", 16, 1024, 14336, False, False, True),
+    ("decode exchange tree, bf16", "0", 32, 1024, 4096, True, False, True),
+    ("decode exchange tree, act-order", "0", 16, 1024, 28672, False, True, True),
+    ("prefill unsplit, exact scaling", "0", 4096, 4096, 14336, False, False, False),
+    ("prefill K slices + combine", "0", 256, 4096, 14336, False, False, True),
+    ("kwave unsplit", "2,64,1", 200, 1096, 14336, False, False, False),
+    ("kwave unsplit, bf16, act-order", "1,128,1", 40, 1024, 14336, True, True, False),
+    ("kwave K slices", "2,128,4", 100, 1024, 28672, False, False, True),
+    ("kwave K slices, bf16", "1,32,8", 31, 520, 28672, True, False, True),
 ]
 
 
-@pytest.mark.parametrize("name,m,n,k,bf16,act,ws_expected", DEFAULT_PLAN_CASES)
-def test_pre_cast_accumulators_default_plans(env, name, m, n, k, bf16, act, ws_expected):
+def _plans(lib, bf16, act, m, n, k):
+    """What the library describes for the call: the medium-M plan or "none", and the other."""
+    lib.pw4_medium_plan_describe.argtypes = lib.pw4_plan_describe.argtypes
+    buf, out = ctypes.create_string_buffer(160), []
+    for describe in (lib.pw4_medium_plan_describe, lib.pw4_plan_describe):
+        assert describe(1, DTYPE_BF16 if bf16 else DTYPE_F16, DTYPE_F16 if act else DTYPE_F32, int(act), int(act), 0,
+                        m, n, k, G, 0, buf, len(buf)) == 0
+        out.append(buf.value.decode())
+    return out
+
+
+@pytest.mark.parametrize("name,kwave,m,n,k,bf16,act,ws_expected", DEFAULT_PLAN_CASES)
+def test_pre_cast_accumulators_default_plans(env, monkeypatch, name, kwave, m, n, k, bf16, act, ws_expected):
     lib, hip = env
     what = f"{name}: M={m} N={n} K={k} {'bf16' if bf16 else 'fp16'}"
     print(what, flush=True)
+    monkeypatch.setenv("PW4_KWAVE", kwave)
+    medium, other = _plans(lib, bf16, act, m, n, k)
+    if kwave == "0":
+        assert medium == "none" and other.startswith(name.split()[0]), (medium, other)
+        assert (" tree=1" in other) == ("exchange tree" in name), other
+    else:
+        rt, nb, splits = kwave.split(",")
+        assert medium == f"kwave rows={32 * int(rt)} nb={nb} splits={splits}", medium
     p = O.make_problem(m, n, k, G, seed=m + 3 * n + k, bf16=bf16, symmetric=not act, act_order=act)
     wm = hip.malloc(lib.pw4_marlin_words(n, k) * 4)
     if act:
@@ -141,10 +167,10 @@ def test_pre_cast_accumulators_default_plans(env, name, m, n, k, bf16, act, ws_e
     y32 = hip.malloc(m * n * 4)
     hip.memset(y32, 0xFF, m * n * 4)  # NaN everywhere: an element the call does not write fails below
     ws_bytes = lib.pw4_gemm_w4a16_marlin_workspace_size(m, n, k, G, int(act), 0)
-    # the plan is the one named: the exchange tree and K slices use the workspace's zero region
-    # and partials; the direct store and the unsplit prefill use none (act-order's copy of x
-    # takes a workspace either way)
-    if not act:
+    # the exchange tree and K slices use the workspace's zero region and partials; the direct
+    # store and the unsplit prefill use none (act-order's copy of x takes a workspace either
+    # way, and the size is the larger of a medium-M call's two plans)
+    if not act and (kwave == "0" or ws_expected):
         assert (ws_bytes > 0) == ws_expected, (what, ws_bytes)
     ws = hip.malloc(max(ws_bytes, 1))
     hip.memset(ws, 0, max(ws_bytes, 1))

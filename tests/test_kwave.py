@@ -67,12 +67,16 @@ CASES = [
     ("2,96,1", 63, 520, 768, 128),
     ("2,112,5", 130, 904, 2560, 128),
     ("2,128,8", 48, 136, 8192, 128),
+    ("1,64,1", 33, 256, 1152, 192),   # three chunks a group: the group index of a chunk is no shift
+    ("2,128,2", 70, 264, 3840, 192),
+    ("1,32,3", 24, 72, 2560, 320),
 ]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("sdtype,sym,act", [(torch.float16, True, False), (torch.float32, False, True)])
+@pytest.mark.parametrize("sdtype,sym,act", [(torch.float16, True, False), (torch.float32, False, True),
+                                            (torch.float16, False, True), (torch.float32, True, False)])
 @pytest.mark.parametrize("plan,m,n,k,g", CASES)
 def test_kwave_plans(pin, plan, m, n, k, g, dtype, sdtype, sym, act):
     c = baseline_case(m, n, k, g, dtype=dtype, seed=m * 3 + n, symmetric=sym, act_order=act)
@@ -81,6 +85,78 @@ def test_kwave_plans(pin, plan, m, n, k, g, dtype, sdtype, sym, act):
     check(y, c.y_ref, dtype, f"{plan} m={m} n={n} k={k} g={g} {dtype}")
     for _ in range(3):  # the counters are left zero, and the sum does not depend on arrival
         assert torch.equal(_run(c, g, sdtype, act, sym), y)
+
+
+def _silu(y):
+    t = y.astype(np.float64).reshape(y.shape[0], -1, 2, 8)
+    return (t[:, :, 0] / (1.0 + np.exp(-t[:, :, 0])) * t[:, :, 1]).reshape(y.shape[0], -1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sym,act", [(True, False), (False, True)])
+@pytest.mark.parametrize("plan,m,n,k", [("1,32,1", 9, 48, 512), ("1,48,1", 31, 208, 1024), ("2,64,2", 65, 320, 2048),
+                                        ("2,112,1", 47, 464, 768), ("1,128,1", 33, 144, 1024),
+                                        ("2,128,3", 130, 912, 2560)])
+def test_kwave_silu(pin, plan, m, n, k, sym, act, dtype):
+    """The gate in the kernel's store, unsplit and behind the sum of K slices; tiles whose last
+    columns, and rows, are past the output."""
+    c = baseline_case(m, n, k, 128, dtype=dtype, seed=m + n, symmetric=sym, act_order=act)
+    wm, perm = ops.repack_w4a16_gptq(c.qweight(), torch.from_numpy(c.g_idx).cuda() if act else None, 128)
+    pin(plan)
+    y = ops.gemm_w4a16_silu_mul(c.x, wm, c.scale(torch.float16, kn=True), None if sym else c.qzeros(),
+                                perm if act else None, 128)
+    assert y.shape == (m, n // 2)
+    check(y, _silu(c.y_ref), dtype, f"{plan} m={m} n={n} k={k} {dtype}", abs_excess=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("plan,m,n,k,g", [("1,32,1", 33, 96, 512, 64), ("2,64,2", 64, 320, 2048, 128),
+                                          ("2,128,1", 130, 520, 1088, 64), ("1,128,3", 48, 136, 4096, 128)])
+def test_kwave_packed(pin, plan, m, n, k, g, dtype):
+    """Packed weights past the decode sizes: repacked into the workspace, behind the partial tiles."""
+    c = baseline_case(m, n, k, g, dtype=dtype, seed=m + k)
+    pin(plan)
+    assert describe(m, k, n, g, layout=0).endswith("repack")
+    y = ops.gemm_w4a16(c.x, c.ct_packed(), c.scale(), g)
+    check(y, c.y_ref, dtype, f"{plan} m={m} n={n} k={k} g={g} {dtype}")
+    assert torch.equal(ops.gemm_w4a16(c.x, c.ct_packed(), c.scale(), g), y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(64, 512, 2048), (16, 512, 1024)])
+def test_workspace_too_small_for_the_slices(pin, monkeypatch, m, n, k):
+    """K slices need scratch; without enough of it the call runs its decode or prefill plan, which
+    here needs none, bit for bit as if the medium-M kernel were kept out."""
+    g = 128
+    c = baseline_case(m, n, k, g, seed=m)
+    wm, _ = ops.repack_w4a16_gptq(c.qweight(), None, g)
+    s = c.scale(torch.float16, kn=True)
+    lib = declare(pulsar_amd.capi())
+    monkeypatch.setenv("PW4_PREFILL_SPLITS", "1")
+
+    def call(nbytes):
+        y = torch.empty(m, n, dtype=torch.float16, device="cuda")
+        ws = torch.zeros(max(nbytes, 1), dtype=torch.uint8, device="cuda")
+        rc = lib.pw4_gemm_w4a16_marlin(c.x.data_ptr(), DTYPE_F16, wm.data_ptr(), s.data_ptr(), DTYPE_F16, None, None,
+                                       y.data_ptr(), m, n, k, g, 0, ws.data_ptr() if nbytes else None, nbytes,
+                                       torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rc == 0, rc
+        return y
+
+    pin("0")
+    assert lib.pw4_gemm_w4a16_marlin_workspace_size(m, n, k, g, 0, 0) == 0
+    other = call(0)
+    pin("2,64,2")
+    need = lib.pw4_gemm_w4a16_marlin_workspace_size(m, n, k, g, 0, 0)
+    assert need > 0
+    full = call(need)
+    check(full, c.y_ref, torch.float16, "on its slices")
+    for nbytes in (need - 256, 1 << 20, 0):
+        assert torch.equal(call(nbytes), other), nbytes
+    assert torch.equal(call(need), full)
 
 
 @pytest.mark.gpu

@@ -1,6 +1,9 @@
 """The plans the library picks for the BASELINE layers, read through pw4_plan_describe
 (host logic only: nothing launches).  Each pinned choice is the measured-faster plan on
-MI355X (256 CUs; graph periods in the comments, us, fp16 x):
+MI355X (256 CUs; graph periods in the comments, us, fp16 x).  These are the decode and prefill
+plans, among themselves: between about M = 9 and 512 the medium-M kernel takes a call away from
+them where it is priced lower (test_what_runs below, and tests/test_kwave.py), and they run
+where it does not apply or PW4_KWAVE=0 keeps it out.
 
 * M = 29..32 on the decode kernel, except Llama-3-70B gate_up (8192 x 57344: M = 32 128
   decode / 118 prefill tile) and down (28672 x 8192: M = 32 69.5 / 61.7), which are faster
@@ -32,7 +35,7 @@ L70 = {"qkv": (8192, 10240), "gate_up": (8192, 57344), "down": (28672, 8192)}
 L70o = {"o": (8192, 8192)}
 OVERRIDES = ("PW4_PREFILL_ROWS", "PW4_PREFILL_SPLITS", "PW4_PREFILL_KHALVES", "PW4_PREFILL_EXACT",
              "PW4_PREFILL_TILE", "PW4_DECODE", "PW4_DECODE_BLOCK_SCALES", "PW4_DECODE_PERM_LDS", "PW4_DECODE_NB",
-             "PW4_DECODE_SPLITS", "PW4_DECODE_WPS", "PW4_DECODE_WIN")
+             "PW4_DECODE_SPLITS", "PW4_DECODE_WPS", "PW4_DECODE_WIN", "PW4_KWAVE")
 
 
 @pytest.fixture(scope="module")
@@ -79,6 +82,31 @@ def test_other_layers_decode_up_to_m32(lib, layer, m):
     model, name = layer.split("_", 1)
     k, n = (L8 if model == "8b" else L70)[name]
     assert plan(lib, m, k, n).startswith("decode"), (layer, m, plan(lib, m, k, n))
+
+
+@pytest.mark.parametrize("layer,runs", [
+    # M =          1         16        24        32        64       256       1024      4096
+    ("8b_qkv", ("decode", "decode", "kwave", "kwave", "kwave", "kwave", "prefill", "prefill")),
+    ("8b_o", ("decode", "decode", "decode", "kwave", "kwave", "kwave", "prefill", "prefill")),
+    ("8b_gate_up", ("decode", "decode", "kwave", "kwave", "kwave", "prefill", "prefill", "prefill")),
+    ("8b_down", ("decode", "decode", "kwave", "kwave", "kwave", "kwave", "prefill", "prefill")),
+    ("70b_qkv", ("decode", "decode", "kwave", "kwave", "kwave", "prefill", "prefill", "prefill")),
+    ("70b_down", ("decode", "decode", "kwave", "kwave", "kwave", "kwave", "prefill", "prefill")),
+])
+def test_what_runs(lib, monkeypatch, layer, runs):
+    """The kernel of an unforced MARLIN call: the medium-M plan where there is one, else the other."""
+    lib.pw4_medium_plan_describe.argtypes = lib.pw4_plan_describe.argtypes
+    model, name = layer.split("_", 1)
+    k, n = (L8 if model == "8b" else L70)[name]
+    got, buf = [], ctypes.create_string_buffer(160)
+    for m in (1, 16, 24, 32, 64, 256, 1024, 4096):
+        assert lib.pw4_medium_plan_describe(LAYOUT_MARLIN, DTYPE_F16, DTYPE_F16, 0, 0, 0, m, n, k, G, 0, buf, 160) == 0
+        medium = buf.value.decode()
+        got.append((plan(lib, m, k, n) if medium == "none" else medium).split()[0].replace("prefill256", "prefill"))
+    assert tuple(got) == runs, got
+    monkeypatch.setenv("PW4_KWAVE", "0")
+    assert lib.pw4_medium_plan_describe(LAYOUT_MARLIN, DTYPE_F16, DTYPE_F16, 0, 0, 0, 64, n, k, G, 0, buf, 160) == 0
+    assert buf.value == b"none"
 
 
 def test_m33_leaves_the_decode_kernel(lib):

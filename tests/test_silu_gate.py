@@ -13,7 +13,8 @@ The reference runs two at::linear calls and at::silu(gate) * up
   kernel unsplit (fp16 and bf16 x) and split (split-K combine), and the
   128 x 128 kernel (pinned through PW4_PREFILL_TILE) unsplit and split; the
   decode K-slice and unsplit 128 x 128 plans gate the GEMM output in a second
-  pass.
+  pass.  The medium-M kernel, which by itself takes some of these sizes, is kept
+  out here (PW4_KWAVE=0); its own gate is in test_kwave.py.
 """
 
 import os
@@ -80,8 +81,10 @@ def _silu_ref(y_full: np.ndarray) -> np.ndarray:
 
 @pytest.fixture
 def plan_env():
-    keys = ("PW4_PREFILL_ROWS", "PW4_PREFILL_SPLITS", "PW4_PREFILL_TILE", "PW4_PREFILL_KHALVES")
+    keys = ("PW4_PREFILL_ROWS", "PW4_PREFILL_SPLITS", "PW4_PREFILL_TILE", "PW4_PREFILL_KHALVES", "PW4_DECODE_WIN",
+            "PW4_KWAVE")
     old = {k: os.environ.get(k) for k in keys}
+    os.environ["PW4_KWAVE"] = "0"
     yield os.environ
     for k, v in old.items():
         if v is None:
@@ -104,8 +107,8 @@ CASES = [
     (5, 4160, 256, torch.float16, {}, True),     # N past a 64-column block boundary
     (24, 512, 4096, torch.float16, {}, False),   # decode, exchange-tree K slices
     (32, 256, 28672, torch.float16, {"PW4_DECODE_WIN": "0"}, False),  # decode, counter K slices
-    (32, 256, 28672, torch.float16, {}, False),  # decode, K windows where it would take the counter
-    (48, 256, 4096, torch.float16, {}, False),   # 128-row prefill tile, then the SiLU pass (M > 32)
+    (32, 256, 28672, torch.float16, {}, False),  # the same by default (K windows: test_decode_windows.py)
+    (48, 256, 4096, torch.float16, {}, False),   # 128-row prefill tiles in K slices -> combine (M > 32)
     (300, 1024, 512, torch.float16, {"PW4_PREFILL_SPLITS": "1"}, True),    # 256-wide prefill, unsplit
     (200, 1024, 512, torch.bfloat16, {"PW4_PREFILL_SPLITS": "1"}, False),  # the same, bf16 x
     (129, 512, 2048, torch.float16, {"PW4_PREFILL_SPLITS": "4"}, True),    # 256-wide, K slices -> combine
