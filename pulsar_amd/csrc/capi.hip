@@ -361,11 +361,12 @@ struct KwavePlan {
 // the next wider kernel, for the same time a chunk and no fewer workgroups, and its x is
 // read by more of them (qkv M = 128 14.4 us at 64 columns, 16.1 at 48).  Of equal plans
 // the widest.
-// The price of the pick has a third part under that root, which the choice among plans
-// is better without: an XCD reads a row tile's x once for the column tiles that its
-// workgroups run side by side (tiles run down the rows first, an eighth of them on each
-// XCD), and the XCDs take 7.5 TB/s of it together.  With few columns and many rows it is
-// the longest: M = 2048, 12288 x 512 58 us, of which the steps are 29; 40 on prefill tiles.
+// The price of the pick has one part more, which the choice among plans is better without:
+// an XCD reads a row tile's x once for the column tiles that its workgroups run side by
+// side (tiles run down the rows first, an eighth of them on each XCD), and the XCDs take
+// 7.5 TB/s of it together.  With few columns and many rows that shows (past half of the
+// rest, as the root of the sum of the squares): M = 2048, 12288 x 512 58 us, of which the
+// steps are 29, and 40 on prefill tiles; M = 1024, 16384 x 768 45.7 and 39.9.
 // max_partial: bytes the partial tiles may take.
 KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_t max_splits, size_t max_partial) {
     constexpr double kStep[2][2][3] = {{{0.57, 0.76, 1.28}, {0.85, 1.15, 1.87}},
@@ -403,7 +404,8 @@ KwavePlan plan_kwave(int64_t M, int64_t N, int64_t K, bool bf16, int cus, int64_
     const double rows = (double)ceil_div(M, 32 * best.rt), tiles = rows * (double)ceil_div(N, best.nb);
     const double shared = std::max(1.0, std::floor(std::min(tiles, (double)cus) / 8.0 / rows));
     const double xcd = tiles * 64.0 * best.rt * (double)K / shared / 7.5e6;
-    best.us += std::cbrt(cubes + xcd * xcd * xcd) - std::cbrt(cubes);
+    const double base = std::cbrt(cubes);
+    if (xcd > 0.5 * base) best.us += std::hypot(base, xcd) - base;
     return best;
 }
 
