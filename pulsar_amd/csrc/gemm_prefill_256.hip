@@ -615,16 +615,19 @@ void launch_variant(const PrefillArgs& a, hipStream_t stream, KernelEvents ev) {
         return;
     }
     if (a.tile_rows == TM / 2) {  // every tile 128 rows: twice the workgroups, two per CU
-        // With a second round of pairs that is more than half full, every second run of `cus`
-        // workgroups (the later of a CU's two, in the first round) issues ahead: the pairs end,
-        // and begin their second round, at different times.  776 to 1024 workgroups on 256
-        // CUs, fp16 and bf16, both scale types: 1-6% faster from 16 chunks on (gate_up M =
-        // 1024 229 -> 221.5 us, 1408 x 20000 235 -> 225.6), at 8 chunks 5% faster to 3%
-        // slower.  Up to 768 workgroups it is within 1% either way; past 1024 it was 17%
-        // slower (1232 and 1280 workgroups at 8 chunks) to 4% faster (1344), and on K slices
-        // 7% slower (2048 x 6144 x 14336 on four), so those run without.
-        const int64_t cus = a.cus;
-        w.ahead = tiles128 > 3 * cus && tiles128 <= 4 * cus && a.nchunks >= 16 ? a.cus : 0;
+        // Where the last of several rounds of pairs is more than half full, every second run
+        // of `cus` workgroups (the later of a CU's two, in the first round) issues ahead: the
+        // pairs end, and begin their next round, at different times.  Graph periods, fp16 and
+        // bf16, both scale types, 256 CUs: 776 to 1024 workgroups 1-6% faster from 16 chunks
+        // on (gate_up M = 1024 229 -> 221.5 us, 1408 x 20000 235 -> 225.6), 1312 to 2408
+        // 1-3%, 3584 0-1.4% (gate_up M = 4096 775 -> 767).  It wants eight chunks a round:
+        // below, 3% slower (1024 workgroups at 8 chunks) and 2% (3584 at 16).  With a last
+        // round of half or less it was up to 17% slower (1232 and 1280 at 8 chunks, 2-4% at
+        // 16 to 64), on K slices 7% (2048 x 6144 x 14336 on four), and with one round
+        // nothing, so those run without.
+        const int64_t pair = 2 * (int64_t)a.cus, rounds = a.cus > 0 ? ceil_div(tiles128, pair) : 1;
+        const int64_t last = tiles128 - (rounds - 1) * pair;
+        w.ahead = rounds > 1 && last > a.cus && a.nchunks >= 8 * rounds ? a.cus : 0;
         half(dim3((unsigned)tiles128), w, ev.start, ev.stop, std::false_type{});
         return;
     }

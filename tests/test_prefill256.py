@@ -106,11 +106,12 @@ def test_prefill_tail_split(plan_env):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("m,k", [(3072, 1024), (3200, 1024), (3200, 960), (4096, 1024), (4224, 1024)])
-def test_prefill_second_round_of_pairs(plan_env, m, k, dtype):
-    """768, 800, 1024 and 1056 unsplit 128-row tiles: on 256 CUs both sides of the grids whose
-    second workgroup of each CU issues ahead, and 15 chunks, which do not.  Every fourth row
-    of each 128-row tile against the oracle."""
+@pytest.mark.parametrize("m,k", [(3072, 1024), (3200, 1024), (3200, 960), (4096, 1024), (4224, 1024), (5248, 1536),
+                                 (6144, 1536)])
+def test_prefill_rounds_of_pairs(plan_env, m, k, dtype):
+    """768, 800, 1024, 1056, 1312 and 1536 unsplit 128-row tiles: on 256 CUs both sides of the
+    grids whose second workgroup of each CU issues ahead, and 15 chunks, which do not.  Every
+    fourth row of each 128-row tile against the oracle."""
     plan_env["PW4_PREFILL_ROWS"] = "128"
     plan_env["PW4_PREFILL_SPLITS"] = "1"
     n, g = 8192, 64
