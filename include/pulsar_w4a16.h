@@ -227,9 +227,9 @@ int pw4_gemm_w4a16_silu_mul(const void* x, int x_dtype, const int32_t* weight_ma
  *
  * pw4_gidx_to_perm: perm = stable argsort(g_idx) for an act-order checkpoint.
  *   g_idx [K] int32 group id of each input row; every group must hold exactly
- *   group_size rows.  status_dev is an int32 device word the call zeroes and
- *   then sets nonzero if g_idx is not such a grouping (read it after the stream
- *   syncs: nonzero means PW4_ERR_GIDX).
+ *   group_size rows.  status_dev is an int32 word, in device or pinned host
+ *   memory, that the call stores: 0, or nonzero if g_idx is not such a grouping
+ *   (read it after the stream syncs: nonzero means PW4_ERR_GIDX).
  * pw4_repack_gptq: qweight int32 [K/8, N] (nibble k%8 of word [k/8, n], unsigned)
  *   -> MARLIN layout; repacked row j is original row perm[j] (perm may be NULL).
  *   GPTQ symmetric nibbles and the reference's MARLIN nibbles are the same bytes,

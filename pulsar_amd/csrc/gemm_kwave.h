@@ -38,19 +38,21 @@
 // and the last to arrive for a tile (arrival counter) sums the slices in slice
 // order, stores y and resets the counter.
 //
-// What bounds it.  At M = 32 and 64 on large layers the weight stream (gate_up
-// 4096 x 28672 at M = 32: 10.2 us for the stream alone, 3.3 for the x copies, about
-// 5 for the arithmetic, 1.8 for the sum in LDS, 19 together); LDS copies move 32
-// bytes a clock per CU and return in order with the weights, so x costs as much
-// as weights do, which is why tiles are as wide as the registers allow.  With
-// more row tiles, the arithmetic: 8 VALU and 2 MFMAs per fragment at RT = 2.
+// What bounds it.  At M = 32 the weight stream beside the x copies: LDS copies move 32
+// bytes a clock per CU and return in order with the weights, so x costs as much as
+// weights do, which is why tiles are as wide as the registers allow (gate_up
+// 4096 x 28672: 18.6 us, of which the MFMAs fill 22% of the SIMDs' time and VALU issue
+// 44%).  With two row tiles, and bf16's exact dequant, the issue itself: gate_up M = 64
+// 37% and 47% with fp16 x, 29% and 70% with bf16.
 // Graph periods on one MI355X, fp16 x, us, before (decode kernel up to M = 32,
 // 128-row prefill tiles past it, with their combine) / this kernel:
-//   gate_up 4096 x 28672   M = 32 29.0 / 19.9, M = 64 41.5 / 24.9, M = 128 43.9 / 43.7
-//   down 14336 x 4096      M = 32 24.3 / 14.9, M = 64 33.0 / 19.6, M = 256 45.9 / 41.0
-//   qkv 4096 x 6144        M = 32 11.4 / 9.6, M = 64 22.0 / 11.5, M = 256 28.3 / 20.9
-//   o 4096 x 4096          M = 64 19.0 / 9.2, M = 256 23.7 / 14.4, M = 512 30.2 / 22.9
-//   70B down 28672 x 8192  M = 32 61.5 / 33.8, M = 64 63.8 / 44.5
+//   gate_up 4096 x 28672   M = 24 27.0 / 18.1, M = 32 29.2 / 18.7, M = 64 42.6 / 24.2
+//   down 14336 x 4096      M = 32 24.3 / 13.6, M = 64 31.8 / 18.1, M = 256 43.4 / 39.8
+//   qkv 4096 x 6144        M = 32 11.0 / 9.2, M = 64 21.1 / 10.8, M = 256 27.5 / 20.2
+//   o 4096 x 4096          M = 64 18.8 / 8.6, M = 256 24.3 / 14.0, M = 512 31.5 / 23.0
+//   70B down 28672 x 8192  M = 32 64.8 / 34.3, M = 64 68.5 / 45.0
+//   70B gate_up 8192 x 57344  M = 20 95.9 / 57.0, M = 32 125 / 62.4
+// bf16 x: gate_up M = 64 41.9 / 26.9, down M = 64 35.0 / 19.0, qkv M = 256 27.7 / 24.2.
 //
 // Reference counterpart: w4a16_marlin_kernel at BM = 32 and 64
 // (pulsar-core/src/kernels/w4a16_marlin.cu:197-304).
