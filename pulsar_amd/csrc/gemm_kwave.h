@@ -29,10 +29,10 @@
 //
 // Range.  The running sum is y / s_g, which fp32 does not hold for every input that
 // y fits: scales far apart or (bf16) very large x overflow it.  A workgroup whose sums
-// come out infinite or NaN computes its slice again, each chunk's products scaled by
-// themselves, and a scale out of range (scale_in_range) makes them NaN.  fp16 x cannot get
-// there within that range, so fp16 x with fp16 scales has no check; the others look behind
-// their stores.
+// come out infinite or NaN where x is finite computes its slice again, each chunk's
+// products scaled by themselves, and a scale out of range (scale_in_range) makes them
+// NaN.  fp16 x cannot get there within that range, so fp16 x with fp16 scales has no
+// check; the others look behind their stores.
 //
 // K slices across workgroups (small N): every workgroup writes its fp32 tile
 // and the last to arrive for a tile (arrival counter) sums the slices in slice
@@ -111,7 +111,8 @@ void kwave_kernel(const KwaveArgs a) {
     __shared__ __attribute__((aligned(256))) uint8_t ss1[kWaves * kScaleSlot];
     __shared__ __attribute__((aligned(256))) uint8_t ss2[D > 2 ? kWaves * kScaleSlot : 16];
     __shared__ __attribute__((aligned(256))) uint8_t ss3[D > 2 ? kWaves * kScaleSlot : 16];
-    __shared__ int s_bad, s_last;
+    __shared__ int s_last, s_over;
+    __shared__ uint32_t s_bad[RT];  // rows whose sums are infinite or NaN
     auto xs = [&](auto i) -> uint8_t* {
         constexpr int I = decltype(i)::value;
         if constexpr (I == 0) return xs0;
@@ -403,8 +404,7 @@ void kwave_kernel(const KwaveArgs a) {
     // and its lane index anew, or the compiler holds what it derives from them in registers
     // through the whole slice: bf16 x, fp32 scales, zero points, gate_up M = 64 30.6 -> 33.1 us.
     auto rescan = [&]() {
-        const KwaveArgs* p = reinterpret_cast<const KwaveArgs*>(
-            (const void*)__builtin_amdgcn_kernarg_segment_ptr());
+        const KwaveArgs* p = reinterpret_cast<const KwaveArgs*>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
         asm volatile("" : "+s"(p));
         int ln = threadIdx.x;
         asm volatile("" : "+v"(ln));
@@ -487,7 +487,8 @@ void kwave_kernel(const KwaveArgs a) {
     };
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_s_waitcnt(0);  // this wave's copies into LDS are done (those past its chunks too)
-    if (tid == 0) s_bad = 0;
+    if (tid < RT) s_bad[tid] = 0;
+    if (tid == 0) s_over = 0;
     constexpr int kQuads = RT * C * 256;
     constexpr int QT = (kQuads + kThreads - 1) / kThreads;  // quads per thread
     f32x4 sum[QT];
@@ -583,14 +584,55 @@ void kwave_kernel(const KwaveArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) bad |= !(__builtin_fabsf(sum[i][e]) <= 0x1.fffffep127f);
         }
-        if (__ballot(bad) != 0 && lane == 0) s_bad = 1;
+        if (__builtin_expect(__ballot(bad) != 0, 0)) {
+#pragma unroll
+            for (int i = 0; i < QT; ++i) {
+                const int q = tid + i * kThreads;
+                if (kQuads % kThreads != 0 && q >= kQuads) break;
+                uint32_t rows4 = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rows4 |= (uint32_t)!(__builtin_fabsf(sum[i][e]) <= 0x1.fffffep127f) << e;
+                if (rows4) atomicOr(&s_bad[q / (C * 256)], rows4 << (8 * ((q >> 6) & 3) + 4 * ((q & 63) >> 5)));
+            }
+        }
+    };
+    // Whether a row of s_bad is finite in x (an infinity or NaN of x belongs in its row's
+    // sums, and is there already).  Every wave looks at every eighth row.
+    auto overflowed = [&]() {
+        constexpr uint32_t kInf = BF16 ? 0x7f80u : 0x7c00u;
+        const KwaveArgs* p = reinterpret_cast<const KwaveArgs*>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
+        asm volatile("" : "+s"(p));
+        int ln = threadIdx.x;
+        asm volatile("" : "+v"(ln));
+        const int begin = split * p->chunks_per_split, end = min(begin + p->chunks_per_split, p->nchunks);
+#pragma unroll 1
+        for (int r = __builtin_amdgcn_readfirstlane(ln >> 6); r < 32 * RT; r += kWaves) {
+            if (!((s_bad[r >> 5] >> (r & 31)) & 1u) || m0 + r >= p->M) continue;
+            const u32x4* xr = reinterpret_cast<const u32x4*>(p->x + (int64_t)(m0 + r) * p->K);
+            bool inf = false;
+#pragma unroll 1
+            for (int i = begin * 8 + (ln & 63); i < end * 8; i += 64) {
+                const u32x4 v = xr[i];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) inf |= (v[j] & kInf) == kInf || ((v[j] >> 16) & kInf) == kInf;
+            }
+            if (__ballot(inf) == 0 && (ln & 63) == 0) s_over = 1;
+        }
+        __syncthreads();  // (s_bad stays as it is: a wave may still be at its any_bad)
+        return __builtin_amdgcn_readfirstlane(s_over) != 0;
+    };
+    auto any_bad = [&]() {
+        uint32_t v = 0;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) v |= s_bad[rt];
+        return __builtin_amdgcn_readfirstlane(v) != 0;
     };
     if (a.partial == nullptr) {
         store_sums();
         if constexpr (kCheck) {
             look();
             __syncthreads();  // (and every wave has read the regions)
-            if (__builtin_expect(s_bad, 0)) {
+            if (__builtin_expect(any_bad(), 0) && overflowed()) {
                 rescan();
                 add_waves();
                 store_sums();
@@ -623,7 +665,7 @@ void kwave_kernel(const KwaveArgs a) {
     };
     write_part();
     if constexpr (kCheck) {
-        if (__builtin_expect(s_bad, 0)) {
+        if (__builtin_expect(any_bad(), 0) && overflowed()) {
             rescan();
             add_waves();
             write_part();

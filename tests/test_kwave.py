@@ -237,6 +237,36 @@ def test_large_bf16_activations(pin, plan, sdtype, sym):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("plan", ["1,64,1", "2,128,2"])
+def test_overflow_beside_rows_that_are_infinite_by_themselves(pin, plan):
+    """Rows whose x holds an infinity or NaN need no second look; rows that overflow beside them
+    do, in the same tile and in others, for large bf16 x and for scales far apart."""
+    m, n, k, g = 72, 256, 2048, 128
+    bad = {3: float("inf"), 40: float("nan"), 71: float("-inf")}
+    keep = [i for i in range(m) if i not in bad]
+    pin(plan)
+    for dtype in (torch.bfloat16, torch.float16):
+        c = baseline_case(m, n, k, g, dtype=dtype, seed=31)
+        if dtype == torch.bfloat16:
+            c.x = (c.x.float() * 2.0 ** 121).to(dtype)
+            for row, v in bad.items():
+                c.x[row, 17 * row] = v
+            y = _run(c, g, torch.float16, False, True)
+            check(y[keep].double() * 2.0 ** -121, c.y_ref[keep], dtype, f"{plan} large x")
+            assert not y[list(bad)].isfinite().any()
+            c = baseline_case(m, n, k, g, dtype=dtype, seed=31)
+        s = np.full_like(c.scale_nk, 16.0)
+        s[:, 5] = 2.0 ** -119
+        c.scale_nk = s
+        ref = _ref64(c, g)
+        for row, v in bad.items():
+            c.x[row, 17 * row] = v
+        y = _run(c, g, torch.float32, False, True)
+        check(y[keep], ref[keep], dtype, f"{plan} {dtype} scales", abs_excess=False)
+        assert not y[list(bad)].isfinite().any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_infinite_and_nan_rows_stay_in_their_rows(pin, dtype):
     m, n, k, g = 48, 192, 1024, 128
